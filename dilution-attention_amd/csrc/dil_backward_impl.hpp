@@ -51,10 +51,11 @@ namespace dil {
 namespace {
 
 struct BwdParams {
-  const void* q;      // CT rows (n, T, D)
+  const void* q;      // CT rows, T per slice
   const void* k;
   const void* v;
-  const void* dout;   // CT rows
+  RowsView qv, kv, vv;
+  const void* dout;   // dO': CT rows (n, T, D)
   const void* qt;     // CT transposed copies, tile-major (T_pad rows per slice)
   const void* kt;
   const void* dot;
@@ -76,6 +77,7 @@ struct BwdParams {
   void* dq;
   void* dk;
   void* dv;
+  RowsView gqv, gkv, gvv;   // where their rows go
   int gdt;            // grad dtype
   int lpt;            // dispatch longest first (xcd_work_item)
 };
@@ -84,7 +86,7 @@ struct BwdParams {
 // per-row prologue
 
 template <typename CT, int D, int BID = BID_SOFTMAX>
-__global__ __launch_bounds__(kThreads) void bwd_rows(const void* __restrict__ dout, int ddt,
+__global__ __launch_bounds__(kThreads) void bwd_rows(const void* __restrict__ dout, RowsView dov, int ddt,
                                                      const float* __restrict__ out,
                                                      const float* __restrict__ rmax,
                                                      const float* __restrict__ rden,
@@ -109,7 +111,7 @@ __global__ __launch_bounds__(kThreads) void bwd_rows(const void* __restrict__ do
     float acc = 0.f;
     if (ok) {
       float o[8];
-      load8_f32(dout, row * D + c8, ddt, v);
+      load8_f32(dout, dov.slice(slice) + (r0 + r) * dov.sr + c8, ddt, v);
       load8_f32(out, row * D + c8, DT_F32, o);
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc = fmaf(v[e], o[e], acc);
@@ -254,7 +256,7 @@ constexpr int query_waves() {
 // products run over all D).  The first of them stores the suffix checkpoints.
 template <typename CT, int D> constexpr int key_split() { return D > 128 ? 2 : 1; }
 
-template <typename CT, int D, int BID = BID_SOFTMAX, int SHARE = SHARE_INCL>
+template <typename CT, int D, int BID = BID_SOFTMAX, int SHARE = SHARE_INCL, bool FLAT = true>
 __global__ __launch_bounds__(kThreads, (bwd_occupancy<CT, D>())) void bwd_key(BwdParams P) {
   using TL = Tiles<CT, D>;
   constexpr int kSplit = key_split<CT, D>();
@@ -285,7 +287,7 @@ __global__ __launch_bounds__(kThreads, (bwd_occupancy<CT, D>())) void bwd_key(Bw
   const int nq = static_cast<int>((P.T + kTileQ - 1) / kTileQ);
   const bool active = static_cast<int64_t>(kb) * kTileK < P.T;
 
-  const CT* qs = static_cast<const CT*>(P.q) + slice * P.T * D;
+  const CT* qs = static_cast<const CT*>(P.q) + P.qv.slice(slice);
   const CT* dos = static_cast<const CT*>(P.dout) + slice * P.T * D;
   const CT* qts = static_cast<const CT*>(P.qt) + slice * D * P.t_pad;
   const CT* dots = static_cast<const CT*>(P.dot) + slice * D * P.t_pad;
@@ -295,8 +297,8 @@ __global__ __launch_bounds__(kThreads, (bwd_occupancy<CT, D>())) void bwd_key(Bw
   // this wave's keys as B operands (lane <-> key)
   RowFrag<CT, D> kf, vf;
   if (key < P.T) {
-    load_row_frag<CT, D>(kf, static_cast<const CT*>(P.k) + (slice * P.T + key) * D + h * (D / 2));
-    load_row_frag<CT, D>(vf, static_cast<const CT*>(P.v) + (slice * P.T + key) * D + h * (D / 2));
+    load_row_frag<CT, D>(kf, static_cast<const CT*>(P.k) + P.kv.slice(slice) + key * P.kv.sr + h * (D / 2));
+    load_row_frag<CT, D>(vf, static_cast<const CT*>(P.v) + P.vv.slice(slice) + key * P.vv.sr + h * (D / 2));
   } else {
     zero_row_frag<CT, D>(kf);
     zero_row_frag<CT, D>(vf);
@@ -313,7 +315,8 @@ __global__ __launch_bounds__(kThreads, (bwd_occupancy<CT, D>())) void bwd_key(Bw
 
   // a stage: the Q and dO' row tiles, their transposes, the row statistics and
   // the demand checkpoints of the workgroup's 128 keys entering the tile
-  KTileLoader<CT, D, true> ql, dl;        // row tiles in query-split slot order
+  KTileLoader<CT, D, true, kLoadBuffer, FLAT> ql;   // row tiles in query-split slot order
+  KTileLoader<CT, D, true> dl;
   TTileLoader<CT, kDH, kLoadBuffer, D> qtl, dtl;   // head dims [t0 * 32, t0 * 32 + kDH) of the transposes
   RowStatsLoader<kNS> sl;
   if constexpr (!bid_log2<BID>()) sl.pad0 = 0.f;
@@ -324,8 +327,8 @@ __global__ __launch_bounds__(kThreads, (bwd_occupancy<CT, D>())) void bwd_key(Bw
   const int64_t t_off = static_cast<int64_t>(t0) * 32 * kTileK;   // the first taken head dim within a tile
   auto fetch = [&](int qt) {
     const int64_t row0 = static_cast<int64_t>(qt) * kTileQ;
-    ql.load(qs, row0, P.T);
-    dl.load(dos, row0, P.T);
+    ql.load(qs, row0, P.T, P.qv.sr);
+    dl.load(dos, row0, P.T, D);
     qtl.load(qts + t_off, row0);
     dtl.load(dots + t_off, row0);
     sl.load(lse, dbs, BID == BID_SOFTMAX ? dbs : P.rb1 + slice * P.T, row0, P.T);
@@ -480,7 +483,7 @@ __global__ __launch_bounds__(kThreads, (bwd_occupancy<CT, D>())) void bwd_key(Bw
   if (key < P.T) {
     // registers 4 j .. 4 j + 3 hold four consecutive head dims (acc_row)
     float* dkrow = P.dkm + (slice * P.T + key) * D;
-    const int64_t dvrow = (slice * P.T + key) * D;
+    const int64_t dvrow = P.gvv.slice(slice) + key * P.gvv.sr;
 #pragma unroll
     for (int t = 0; t < kDT; ++t)
 #pragma unroll
@@ -500,7 +503,7 @@ __global__ __launch_bounds__(kThreads, (bwd_occupancy<CT, D>())) void bwd_key(Bw
 // row-parallel dq pass
 
 template <typename CT, int D, int BID = BID_SOFTMAX, int SHARE = SHARE_INCL, bool PARK = false,
-          int W = 4>
+          int W = 4, bool FLAT = true>
 __global__ __launch_bounds__(64 * W, ((PARK && query_parks<CT, D>()) ? (W == 4 ? 3 : 1) : bwd_occupancy<CT, D>())) void bwd_query(
     BwdParams P) {
   using TL = Tiles<CT, D>;
@@ -537,15 +540,15 @@ __global__ __launch_bounds__(64 * W, ((PARK && query_parks<CT, D>()) ? (W == 4 ?
   const int nkt_wg = static_cast<int>((wg_last + kTileK - 1) / kTileK);
   const int nkt_w = r0 < P.T ? qt + 1 : 0;
 
-  const CT* ks = static_cast<const CT*>(P.k) + slice * P.T * D;
-  const CT* vs = static_cast<const CT*>(P.v) + slice * P.T * D;
+  const CT* ks = static_cast<const CT*>(P.k) + P.kv.slice(slice);
+  const CT* vs = static_cast<const CT*>(P.v) + P.vv.slice(slice);
   const CT* kts = static_cast<const CT*>(P.kt) + slice * D * P.t_pad;
 
   // this wave's rows in QS order: register i of half h <-> row r0 + 16 h + i
   RowFrag<CT, D> qf, dof;
   const int64_t my_row = r0 + qsig(l32);
   if (my_row < P.T) {
-    load_row_frag<CT, D>(qf, static_cast<const CT*>(P.q) + (slice * P.T + my_row) * D + h * (D / 2));
+    load_row_frag<CT, D>(qf, static_cast<const CT*>(P.q) + P.qv.slice(slice) + my_row * P.qv.sr + h * (D / 2));
     load_row_frag<CT, D>(dof, static_cast<const CT*>(P.dout) + (slice * P.T + my_row) * D + h * (D / 2));
   } else {
     zero_row_frag<CT, D>(qf);
@@ -738,14 +741,14 @@ __global__ __launch_bounds__(64 * W, ((PARK && query_parks<CT, D>()) ? (W == 4 ?
   // the end (both measured best for their form)
   // the tile loaders are laid out for kThreads threads: with 8 waves, waves
   // 0-3 stage the tiles that all 8 read (a wave-uniform condition)
-  KTileLoader<CT, D, false, kPark ? kLoadBuffer : kLoadSkip> kl, vl;
+  KTileLoader<CT, D, false, kPark ? kLoadBuffer : kLoadSkip, FLAT> kl, vl;
   TTileLoader<CT, D, kPark ? kLoadBuffer : kLoadClamp> ktl;
   const bool stager = W == 4 || threadIdx.x < kThreads;
   auto fetch = [&](int kt) {
     if (!stager) return;
     const int64_t key0 = static_cast<int64_t>(kt) * kTileK;
-    kl.load(ks, key0, P.T);
-    vl.load(vs, key0, P.T);
+    kl.load(ks, key0, P.T, P.kv.sr);
+    vl.load(vs, key0, P.T, P.vv.sr);
     ktl.load(kts, key0);
   };
   auto stash = [&](int buf) {
@@ -801,7 +804,7 @@ __global__ __launch_bounds__(64 * W, ((PARK && query_parks<CT, D>()) ? (W == 4 ?
     const int row = acc_row(i, h);
     if (r0 + row < P.T) {
       const float gr = g_s[wave][row];
-      const int64_t base = (slice * P.T + r0 + row) * D;
+      const int64_t base = P.gqv.slice(slice) + (r0 + row) * P.gqv.sr;
 #pragma unroll
       for (int t = 0; t < kDTiles<D>; ++t) {
         const int d = 32 * t + l32;
@@ -817,7 +820,7 @@ __global__ __launch_bounds__(64 * W, ((PARK && query_parks<CT, D>()) ? (W == 4 ?
 // ---------------------------------------------------------------------------
 // softmax-Jacobian correction of dk
 
-template <typename CT, int D, int BID = BID_SOFTMAX>
+template <typename CT, int D, int BID = BID_SOFTMAX, bool FLAT = true>
 __global__ __launch_bounds__(kThreads, (sizeof(CT) == 2 && D <= 64) ? 3 : 2) void bwd_dkcorr(BwdParams P) {
   using TL = Tiles<CT, D>;
   constexpr int kSplit = key_split<CT, D>();          // head-dim split as in bwd_key
@@ -845,25 +848,25 @@ __global__ __launch_bounds__(kThreads, (sizeof(CT) == 2 && D <= 64) ? 3 : 2) voi
   const int nq = static_cast<int>((P.T + kTileQ - 1) / kTileQ);
   const bool active = static_cast<int64_t>(kb) * kTileK < P.T;
 
-  const CT* qs = static_cast<const CT*>(P.q) + slice * P.T * D;
+  const CT* qs = static_cast<const CT*>(P.q) + P.qv.slice(slice);
   const CT* qgts = static_cast<const CT*>(P.qgt) + slice * D * P.t_pad;
   const float* lse = P.lse + slice * P.T;
 
   RowFrag<CT, D> kf;
-  if (key < P.T) load_row_frag<CT, D>(kf, static_cast<const CT*>(P.k) + (slice * P.T + key) * D + h * (D / 2));
+  if (key < P.T) load_row_frag<CT, D>(kf, static_cast<const CT*>(P.k) + P.kv.slice(slice) + key * P.kv.sr + h * (D / 2));
   else zero_row_frag<CT, D>(kf);
   floatx16 dkc[kDT];
 #pragma unroll
   for (int t = 0; t < kDT; ++t) dkc[t] = floatx16{};
 
-  KTileLoader<CT, D, true> ql;            // row tile in query-split slot order
+  KTileLoader<CT, D, true, kLoadBuffer, FLAT> ql;   // row tile in query-split slot order
   TTileLoader<CT, kDH, kLoadBuffer, D> qtl;   // the workgroup's head dims of (ghat q)^T
   const int64_t t_off = static_cast<int64_t>(t0) * 32 * kTileK;
   RowStatsLoader<kNS, false> sl;
   if constexpr (!bid_log2<BID>()) sl.pad0 = 0.f;
   auto fetch = [&](int qt) {
     const int64_t row0 = static_cast<int64_t>(qt) * kTileQ;
-    ql.load(qs, row0, P.T);
+    ql.load(qs, row0, P.T, P.qv.sr);
     qtl.load(qgts + t_off, row0);
     sl.load(lse, lse, BID == BID_SOFTMAX ? lse : P.rb1 + slice * P.T, row0, P.T);
   };
@@ -935,7 +938,7 @@ __global__ __launch_bounds__(kThreads, (sizeof(CT) == 2 && D <= 64) ? 3 : 2) voi
   if (key < P.T) {
     // every dk_main load first (the dk stores could alias them for all the
     // compiler knows), four consecutive head dims per load and store
-    const int64_t base = (slice * P.T + key) * D;
+    const int64_t base = (slice * P.T + key) * D, out = P.gkv.slice(slice) + key * P.gkv.sr;
     floatx4 dm[kDT][4];
 #pragma unroll
     for (int t = 0; t < kDT; ++t)
@@ -953,7 +956,7 @@ __global__ __launch_bounds__(kThreads, (sizeof(CT) == 2 && D <= 64) ? 3 : 2) voi
           floatx4 v;
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = (dm[t][j][e] - dkc[t][4 * j + e]) * P.scale;
-          store4_as(P.dk, base + d, P.gdt, v);
+          store4_as(P.dk, out + d, P.gdt, v);
         }
       }
   }
@@ -991,7 +994,7 @@ __global__ __launch_bounds__(kThreads, (sizeof(CT) == 2 && D <= 64) ? 3 : 2) voi
 #endif
 using KqPart = std::conditional_t<DIL_KEYQ_F32_PARTIALS != 0, float, __bf16>;
 
-template <int D, int BID = BID_SOFTMAX, int SHARE = SHARE_INCL>
+template <int D, int BID = BID_SOFTMAX, int SHARE = SHARE_INCL, bool FLAT = true>
 __global__ __launch_bounds__(kKqThreads, 2) void bwd_keyq(BwdParams P, KqPart* __restrict__ dqp,
                                                            float* __restrict__ ghp, int64_t ntiles) {
   static_assert(D == 64, "the dq-forming key pass is built for head_dim 64");
@@ -1026,7 +1029,7 @@ __global__ __launch_bounds__(kKqThreads, 2) void bwd_keyq(BwdParams P, KqPart* _
   const int nq = static_cast<int>((P.T + kTileQ - 1) / kTileQ);
   const bool active = static_cast<int64_t>(kb) * kTileK < P.T;
 
-  const CT* qs = static_cast<const CT*>(P.q) + slice * P.T * D;
+  const CT* qs = static_cast<const CT*>(P.q) + P.qv.slice(slice);
   const CT* dos = static_cast<const CT*>(P.dout) + slice * P.T * D;
   const CT* qts = static_cast<const CT*>(P.qt) + slice * D * P.t_pad;
   const CT* dots = static_cast<const CT*>(P.dot) + slice * D * P.t_pad;
@@ -1036,8 +1039,8 @@ __global__ __launch_bounds__(kKqThreads, 2) void bwd_keyq(BwdParams P, KqPart* _
   // this wave's keys as B operands (lane <-> key)
   RowFrag<CT, D> kf, vf;
   if (key < P.T) {
-    load_row_frag<CT, D>(kf, static_cast<const CT*>(P.k) + (slice * P.T + key) * D + h * (D / 2));
-    load_row_frag<CT, D>(vf, static_cast<const CT*>(P.v) + (slice * P.T + key) * D + h * (D / 2));
+    load_row_frag<CT, D>(kf, static_cast<const CT*>(P.k) + P.kv.slice(slice) + key * P.kv.sr + h * (D / 2));
+    load_row_frag<CT, D>(vf, static_cast<const CT*>(P.v) + P.vv.slice(slice) + key * P.vv.sr + h * (D / 2));
   } else {
     zero_row_frag<CT, D>(kf);
     zero_row_frag<CT, D>(vf);
@@ -1088,13 +1091,18 @@ __global__ __launch_bounds__(kKqThreads, 2) void bwd_keyq(BwdParams P, KqPart* _
   float cr = 0.f;
   // whole-slice resources, built once: the tile offset advances a 32-bit
   // per-lane offset (rows past T read as zeros through the resource bound)
-  const auto rres = make_rsrc(rsrc, P.T * D * static_cast<int64_t>(sizeof(CT)));
+  const int64_t rld = FLAT || second ? D : P.qv.sr;   // elements per row of the staged row tile's source
+  const auto rres = make_rsrc(rsrc, rows_bytes<CT, D>(P.T, rld));
+  const uint32_t rtile = FLAT ? kTileQ * D * 2u : __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(rld) * (kTileQ * 2u));
+  const uint32_t roff = FLAT ? 0u
+                             : static_cast<uint32_t>(c256 / (D / 8)) * static_cast<uint32_t>(rld) * 2u +
+                                   static_cast<uint32_t>(c256 % (D / 8)) * 16u;
   const auto tres = make_rsrc(tsrc, D * P.t_pad * static_cast<int64_t>(sizeof(CT)));
   auto fetch = [&](int qt) {
     const int64_t row0 = static_cast<int64_t>(qt) * kTileQ;
     const uint32_t off = static_cast<uint32_t>(qt) * static_cast<uint32_t>(kTileQ * D * sizeof(CT)) +
                          static_cast<uint32_t>(c256 * 16);
-    rr = buffer_load16<bf16x8>(rres, off, 0);
+    rr = buffer_load16<bf16x8>(rres, FLAT ? off : static_cast<uint32_t>(qt) * rtile + roff, 0);
     tr = buffer_load16<bf16x8>(tres, off, 0);
     sl.load(lse, dbs, BID == BID_SOFTMAX ? dbs : P.rb1 + slice * P.T, row0, P.T);
     cr = ccol[static_cast<int64_t>(qt) * P.T];
@@ -1339,7 +1347,7 @@ __global__ __launch_bounds__(kKqThreads, 2) void bwd_keyq(BwdParams P, KqPart* _
   if (key < P.T) {
     // registers 4 j .. 4 j + 3 hold four consecutive head dims (acc_row)
     float* dkrow = P.dkm + (slice * P.T + key) * D;
-    const int64_t dvrow = (slice * P.T + key) * D;
+    const int64_t dvrow = P.gvv.slice(slice) + key * P.gvv.sr;
 #pragma unroll
     for (int t = 0; t < kDTiles<D>; ++t)
 #pragma unroll
@@ -1365,7 +1373,7 @@ __global__ __launch_bounds__(kThreads) void bwd_dq_reduce(const KqPart* __restri
                                                           const float* __restrict__ ghp, int64_t ntiles,
                                                           int64_t T, const float* __restrict__ pk,
                                                           const __bf16* __restrict__ qt, int64_t t_pad,
-                                                          void* __restrict__ dq, int gdt, float scale,
+                                                          void* __restrict__ dq, RowsView gqv, int gdt, float scale,
                                                           __bf16* __restrict__ qgt, int64_t slice0) {
   static_assert(D * kTileQ == 8 * kThreads, "one 16-byte chunk of the partial tile per thread");
   __shared__ float sum_s[D][kTileQ + 1];
@@ -1448,7 +1456,7 @@ __global__ __launch_bounds__(kThreads) void bwd_dq_reduce(const KqPart* __restri
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = sum_s[d8 + e][row] * scale;
     }
-    store8_as(dq, o, gdt, v);
+    store8_as(dq, gqv.slice(slice) + grow * gqv.sr + d8, gdt, v);
   }
 }
 
@@ -1540,9 +1548,9 @@ int launch_backward(const BackwardArgs& a) {
   const unsigned tiles64 = static_cast<unsigned>(t_pad / 64);
   slice_batches(a.n, [&](int64_t s0, unsigned ns) {
     PrepJobs qkv{};
-    qkv.job[0] = PrepJob{a.q, sn, qc, sn, qt, nullptr};
-    qkv.job[1] = PrepJob{a.k, sn, kc, sn, kt, nullptr};
-    qkv.job[2] = PrepJob{a.v, sn, vc, sn, nullptr, nullptr};
+    qkv.job[0] = PrepJob{a.q, a.qv, qc, sn, qt, nullptr};
+    qkv.job[1] = PrepJob{a.k, a.kv, kc, sn, kt, nullptr};
+    qkv.job[2] = PrepJob{a.v, a.vv, vc, sn, nullptr, nullptr};
     DIL_TIMED("prep", st, (prep_kernel<CT, D><<<dim3(tiles64, ns, convert ? 3 : 2), kThreads, 0, st>>>(
                               qkv, a.dtype, a.T, D * t_pad, t_pad, s0)));
   });
@@ -1551,6 +1559,10 @@ int launch_backward(const BackwardArgs& a) {
   P.q = convert ? static_cast<const void*>(qc) : a.q;
   P.k = convert ? static_cast<const void*>(kc) : a.k;
   P.v = convert ? static_cast<const void*>(vc) : a.v;
+  const RowsView flat = flat_rows(sn, D);
+  P.qv = convert ? flat : a.qv;
+  P.kv = convert ? flat : a.kv;
+  P.vv = convert ? flat : a.vv;
   P.dout = doc;
   P.qt = qt;
   P.kt = kt;
@@ -1577,19 +1589,27 @@ int launch_backward(const BackwardArgs& a) {
   P.dq = a.dq;
   P.dk = a.dk;
   P.dv = a.dv;
+  P.gqv = a.gqv;
+  P.gkv = a.gkv;
+  P.gvv = a.gvv;
   P.gdt = a.grad_dtype;
   P.lpt = longest_first_for(a.n, a.T);
 
   // row statistics and dO' = dO / (S + eps), row-major and transposed
   slice_batches(a.n, [&](int64_t s0, unsigned ns) {
     DIL_TIMED("bwd_rows", st, (bwd_rows<CT, D, BID><<<dim3(tiles64, ns), kThreads, 0, st>>>(
-                                  a.dout, a.dout_dtype, a.out, a.rmax, a.rden, a.ssum, lse, sinv, dbs,
+                                  a.dout, a.dov, a.dout_dtype, a.out, a.rmax, a.rden, a.ssum, lse, sinv, dbs,
                                   reinterpret_cast<float*>(ws + w.rb1), a.T, t_pad, doc, dot, s0)));
   });
   const int nkt = static_cast<int>((a.T + kTileK - 1) / kTileK);
   P.n = a.n;
+  const bool rows_flat = P.qv.sr == D && P.kv.sr == D && P.vv.sr == D;
+  return with_rows<is_production<BID, SHARE>() && D <= 128>(rows_flat, [&](auto flat_tag) -> int {
+  constexpr bool kFlat = decltype(flat_tag)::value;
   if constexpr (std::is_same_v<CT, __bf16> && D == 64) {
-    if (keyq_eligible(a.n, a.T, D, kOperandPrec<CT>)) {
+    // the pass reads a slice's Q rows through one resource with 32-bit offsets
+    const bool q_fits = a.T * P.qv.sr * static_cast<int64_t>(sizeof(CT)) < (int64_t{1} << 31);
+    if (q_fits && keyq_eligible(a.n, a.T, D, kOperandPrec<CT>)) {
       // one key pass forms dv, dk_main and the dq partials; the reduction
       // finishes dq and writes the (ghat q)^T tiles of the dk correction
       KqPart* dqp = reinterpret_cast<KqPart*>(ws + w.dqp);
@@ -1597,31 +1617,31 @@ int launch_backward(const BackwardArgs& a) {
       const int64_t ntiles = keyq_tiles(a.T);
       P.kgroups = static_cast<int>(keyq_groups(a.T));
       const dim3 gkq(static_cast<unsigned>(xcd_grid(static_cast<int64_t>(P.kgroups) * a.n)));
-      DIL_TIMED("bwd_keyq", st, (bwd_keyq<D, BID, SHARE><<<gkq, kKqThreads, 0, st>>>(P, dqp, ghp, ntiles)));
+      DIL_TIMED("bwd_keyq", st, (bwd_keyq<D, BID, SHARE, kFlat><<<gkq, kKqThreads, 0, st>>>(P, dqp, ghp, ntiles)));
       const unsigned nq = static_cast<unsigned>((a.T + kTileQ - 1) / kTileQ);
       slice_batches(a.n, [&](int64_t s0, unsigned ns) {
         constexpr bool kGhat = bid_normalized<BID>();   // the elementwise bids have no ghat
         DIL_TIMED("bwd_dq_reduce", st,
                   (bwd_dq_reduce<D, kGhat><<<dim3(nq, ns), kThreads, 0, st>>>(dqp, ghp, ntiles, a.T, a.pk, qt, t_pad,
-                                                                             a.dq, a.grad_dtype, P.scale, qgt, s0)));
+                                                                             a.dq, a.gqv, a.grad_dtype, P.scale, qgt, s0)));
       });
       P.kgroups = (nkt + 3) / 4;
       const dim3 gkey(static_cast<unsigned>(xcd_grid(static_cast<int64_t>(P.kgroups) * key_split<CT, D>() * a.n)));
-      DIL_TIMED("bwd_dkcorr", st, (bwd_dkcorr<CT, D, BID><<<gkey, kThreads, 0, st>>>(P)));
+      DIL_TIMED("bwd_dkcorr", st, (bwd_dkcorr<CT, D, BID, kFlat><<<gkey, kThreads, 0, st>>>(P)));
       return static_cast<int>(hipGetLastError());
     }
   }
   P.kgroups = (nkt + 3) / 4;
   // bwd_key and bwd_dkcorr: key groups x head-dim parts x slices
   const dim3 gkeys(static_cast<unsigned>(xcd_grid(static_cast<int64_t>(P.kgroups) * key_split<CT, D>() * a.n)));
-  DIL_TIMED("bwd_key", st, (bwd_key<CT, D, BID, SHARE><<<gkeys, kThreads, 0, st>>>(P)));
+  DIL_TIMED("bwd_key", st, (bwd_key<CT, D, BID, SHARE, kFlat><<<gkeys, kThreads, 0, st>>>(P)));
   constexpr bool kParked = query_parks<CT, D>() && is_production<BID, SHARE>();
   constexpr int kQW = kParked ? query_waves<CT, D>() : 4;     // row tiles (waves) per workgroup
   {
     const int kgroups_key = P.kgroups;
     P.kgroups = (nkt + kQW - 1) / kQW;
     const dim3 gq(static_cast<unsigned>(xcd_grid(static_cast<int64_t>(P.kgroups) * a.n)));
-    DIL_TIMED("bwd_query", st, (bwd_query<CT, D, BID, SHARE, kParked, kQW><<<gq, 64 * kQW, 0, st>>>(P)));
+    DIL_TIMED("bwd_query", st, (bwd_query<CT, D, BID, SHARE, kParked, kQW, kFlat><<<gq, 64 * kQW, 0, st>>>(P)));
     P.kgroups = kgroups_key;
   }
   slice_batches(a.n, [&](int64_t s0, unsigned ns) {
@@ -1629,8 +1649,9 @@ int launch_backward(const BackwardArgs& a) {
               prep_ghat_q<CT, D><<<dim3(static_cast<unsigned>(t_pad / 32), ns), kThreads, 0, st>>>(
                   qt, P.ghat, a.T, t_pad, qgt, s0));
   });
-  DIL_TIMED("bwd_dkcorr", st, (bwd_dkcorr<CT, D, BID><<<gkeys, kThreads, 0, st>>>(P)));
+  DIL_TIMED("bwd_dkcorr", st, (bwd_dkcorr<CT, D, BID, kFlat><<<gkeys, kThreads, 0, st>>>(P)));
   return static_cast<int>(hipGetLastError());
+  });
 }
 
 }  // namespace

@@ -40,12 +40,13 @@ namespace dil {
 namespace {
 
 struct FwdParams {
-  const void* q;          // CT rows (n, C, D), slice stride q_sn
-  int64_t q_sn;
-  const void* k;          // CT rows (n, >= Tk, D), slice stride k_sn
-  int64_t k_sn;
-  const void* v;          // CT rows of V (n, >= Tk, D), slice stride v_sn: the key
-  int64_t v_sn;           // pass parks V from them when set (else from vt)
+  const void* q;          // CT rows, C per slice
+  RowsView qv;
+  const void* k;          // CT rows, >= Tk per slice
+  RowsView kv;
+  const void* v;          // CT rows of V, >= Tk per slice: the key pass
+  RowsView vv;            // parks V from them when set (else from vt)
+  int64_t s0;             // first slice of the views' tensors (key-pass batches)
   const void* vt;         // CT V^T, tile-major (Tk_pad rows per slice)
   const void* kt;         // CT K^T, tile-major, or null
   int64_t t_sn, tk_pad;
@@ -56,8 +57,9 @@ struct FwdParams {
   float c;                // log2(e) / sqrt(D)
   float scale;            // 1 / sqrt(D)
   float shift, lshift;    // SHIFT of the expshift / sigshift bids and log2(SHIFT)
-  float* out;
-  int64_t o_sn;
+  void* out;              // C rows per slice, in odt
+  RowsView ov;
+  int odt;
   float* rmax;
   float* rden;
   float* ssum;
@@ -107,7 +109,7 @@ constexpr float kLazyMax = 8.f;
 // ---------------------------------------------------------------------------
 // row statistics (+ pk) and per-32-row-block column sums of p
 
-template <typename CT, int D, bool PK, int BID = BID_SOFTMAX>
+template <typename CT, int D, bool PK, int BID = BID_SOFTMAX, bool FLAT = true>
 __global__ __launch_bounds__(kThreads, 2) void fwd_stats(FwdParams P) {
   using T = Tiles<CT, D>;
   __shared__ __attribute__((aligned(16))) CT ktile[2][kTileK * T::kKStride];
@@ -122,15 +124,15 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_stats(FwdParams P) {
   const WaveRows W = wave_rows(P, g, wave);
   const int nkt_wg = group_key_tiles(P, g);
 
-  const CT* qs = static_cast<const CT*>(P.q) + slice * P.q_sn;
-  const CT* ks = static_cast<const CT*>(P.k) + slice * P.k_sn;
+  const CT* qs = static_cast<const CT*>(P.q) + P.qv.slice(slice);
+  const CT* ks = static_cast<const CT*>(P.k) + P.kv.slice(slice);
   const CT* kts = PK ? static_cast<const CT*>(P.kt) + slice * P.t_sn : nullptr;
 
   // Q rows in natural order: the B operand of sweep 1 (lane <-> query) and the
   // A operand of sweep 2 (register rows <-> queries)
   RowFrag<CT, D> qf;
   const bool row_ok = W.r0 + l32 < P.C;
-  if (row_ok) load_row_frag<CT, D>(qf, qs + (W.r0 + l32) * D + h * (D / 2));
+  if (row_ok) load_row_frag<CT, D>(qf, qs + (W.r0 + l32) * P.qv.sr + h * (D / 2));
   else zero_row_frag<CT, D>(qf);
   const int my_q = static_cast<int>(W.qa0) + l32;      // query of this lane in sweep 1
 
@@ -143,7 +145,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_stats(FwdParams P) {
     return;
   }
 
-  KTileLoader<CT, D> kl;
+  KTileLoader<CT, D, false, kLoadBuffer, FLAT> kl;
   TTileLoader<CT, D> tl;
 
   // ---- sweep 1: S^T = K Q^T (lane <-> query, registers <-> keys) ----
@@ -235,7 +237,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_stats(FwdParams P) {
     }
   };
 
-  kl.load(ks, 0, P.Tk);
+  kl.load(ks, 0, P.Tk, P.kv.sr);
   if constexpr (PK) tl.load(kts, 0);
   kl.store(ktile[0]);
   if constexpr (PK) tl.store(kttile[0]);
@@ -243,7 +245,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_stats(FwdParams P) {
   auto iter = [&](int kt, int buf) __attribute__((always_inline)) {
     if (kt + 1 < nkt_wg) {
       const int64_t key0n = static_cast<int64_t>(kt + 1) * kTileK;
-      kl.load(ks, key0n, P.Tk);
+      kl.load(ks, key0n, P.Tk, P.kv.sr);
       if constexpr (PK) tl.load(kts, key0n);
     }
     if (kt < W.kfull) stats_step(kt, buf, std::false_type{});
@@ -299,7 +301,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_stats(FwdParams P) {
 // fp64 register, stores it as the checkpoint of every block (the demand
 // entering the block) and finally as the key's total.
 
-template <typename CT, int D, int BID = BID_SOFTMAX>
+template <typename CT, int D, int BID = BID_SOFTMAX, bool FLAT = true>
 __global__ __launch_bounds__(kThreads, (sizeof(CT) == 2 && D <= 64) ? 4 : 2) void fwd_demand(FwdParams P) {
   using T = Tiles<CT, D>;
   constexpr int kRP = BID == BID_SOFTMAX ? 1 : 2;                  // per-row parameters
@@ -327,25 +329,25 @@ __global__ __launch_bounds__(kThreads, (sizeof(CT) == 2 && D <= 64) ? 4 : 2) voi
   const int64_t b_w = first_block(key0);
   const int64_t nb = P.nb;
 
-  const CT* qs = static_cast<const CT*>(P.q) + slice * P.q_sn;
+  const CT* qs = static_cast<const CT*>(P.q) + P.qv.slice(slice);
   const float* rmax = P.rmax + slice * P.C;
   const float* rden = P.rden + slice * P.C;
 
   RowFrag<CT, D> kf;
-  if (key_ok) load_row_frag<CT, D>(kf, static_cast<const CT*>(P.k) + slice * P.k_sn + key * D + h * (D / 2));
+  if (key_ok) load_row_frag<CT, D>(kf, static_cast<const CT*>(P.k) + P.kv.slice(slice) + key * P.kv.sr + h * (D / 2));
   else zero_row_frag<CT, D>(kf);
 
   double run = (P.demand_in != nullptr && key < P.q0 && key_ok)
                    ? static_cast<double>(P.demand_in[slice * P.din_sn + key]) : 0.0;
   float* ccol = P.carry + slice * nb * P.Tk + key;
 
-  KTileLoader<CT, D> ql;
+  KTileLoader<CT, D, false, kLoadBuffer, FLAT> ql;
   float rmax_r = 0.f, rden_r = 1.f;
   bool row_ok = false;
   int64_t it_row0 = 0;                       // first chunk row of the fetched block
   auto fetch = [&](int64_t b) {
     it_row0 = b * kTileQ;
-    ql.load(qs, b * kTileQ, P.C);
+    ql.load(qs, b * kTileQ, P.C, P.qv.sr);
     const int64_t r = b * kTileQ + (threadIdx.x & (kTileQ - 1));
     row_ok = r < P.C;
     rmax_r = rmax[min(r, P.C - 1)];
@@ -431,7 +433,7 @@ __global__ __launch_bounds__(kThreads, (sizeof(CT) == 2 && D <= 64) ? 4 : 2) voi
 // ---------------------------------------------------------------------------
 // output pass
 
-template <typename CT, int D, int BID = BID_SOFTMAX, int SHARE = SHARE_INCL>
+template <typename CT, int D, int BID = BID_SOFTMAX, int SHARE = SHARE_INCL, bool FLAT = true>
 __global__ __launch_bounds__(kThreads, 2) void fwd_out(FwdParams P) {
   using T = Tiles<CT, D>;
   constexpr int kRP = BID == BID_SOFTMAX ? 1 : 2;                  // per-row parameters
@@ -452,14 +454,14 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_out(FwdParams P) {
   const int nkt_wg = group_key_tiles(P, g);
   const int nst = (nkt_wg + 1) / 2;                    // stages of two key tiles
 
-  const CT* qs = static_cast<const CT*>(P.q) + slice * P.q_sn;
-  const CT* ks = static_cast<const CT*>(P.k) + slice * P.k_sn;
+  const CT* qs = static_cast<const CT*>(P.q) + P.qv.slice(slice);
+  const CT* ks = static_cast<const CT*>(P.k) + P.kv.slice(slice);
   const CT* vts = static_cast<const CT*>(P.vt) + slice * P.t_sn;
 
   // Q rows in QS order: accumulator register i of half h <-> row 16 h + i
   RowFrag<CT, D> qf;
   const int64_t my_row = W.r0 + qsig(l32);
-  if (my_row < P.C) load_row_frag<CT, D>(qf, qs + my_row * D + h * (D / 2));
+  if (my_row < P.C) load_row_frag<CT, D>(qf, qs + my_row * P.qv.sr + h * (D / 2));
   else zero_row_frag<CT, D>(qf);
 
   // log2-sum-exp of this wave's rows (the per-row bid parameters of the
@@ -587,13 +589,13 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_out(FwdParams P) {
     }
   };
 
-  KTileLoader<CT, D, false, kLoadClamp> kl[kSets][2];  // clamped global loads: measured faster here
+  KTileLoader<CT, D, false, kLoadClamp, FLAT> kl[kSets][2];  // clamped global loads: measured faster here
   TTileLoader<CT, D, kLoadClamp> vl[kSets][2];
   auto fetch = [&](int st, int set) {
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
       const int64_t key0 = static_cast<int64_t>(2 * st + n) * kTileK;
-      kl[set][n].load(ks, key0, P.Tk);
+      kl[set][n].load(ks, key0, P.Tk, P.kv.sr);
       vl[set][n].load(vts, key0);
     }
     const int64_t key = static_cast<int64_t>(st) * 2 * kTileK + cj;
@@ -642,17 +644,22 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_out(FwdParams P) {
   if (h == 0) ssum_s[wave][l32] = rp.lo + rp.hi;
   __syncthreads();
   if (h == 0 && W.r0 + l32 < P.C) P.ssum[slice * P.C + W.r0 + l32] = ssum_s[wave][l32];
+  // the choice of the output type outside the loop: inside, it cost fwd_out 3%
+  const int64_t out0 = P.ov.slice(slice) + W.r0 * P.ov.sr + l32;
+  auto store_out = [&](auto put) __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int row = acc_row(i, h);
-    if (W.r0 + row < P.C) {
-      const float inv = 1.f / (ssum_s[wave][row] + kEps);
-      float* dst = P.out + slice * P.o_sn + (W.r0 + row) * D;
+    for (int i = 0; i < 16; ++i) {
+      const int row = acc_row(i, h);
+      if (W.r0 + row < P.C) {
+        const float inv = 1.f / (ssum_s[wave][row] + kEps);
 #pragma unroll
-      for (int t = 0; t < kDTiles<D>; ++t)
-        if (32 * t + l32 < D) dst[32 * t + l32] = o[t][i] * inv;
+        for (int t = 0; t < kDTiles<D>; ++t)
+          if (32 * t + l32 < D) put(out0 + row * P.ov.sr + 32 * t, o[t][i] * inv);
+      }
     }
-  }
+  };
+  if (P.odt == DT_F32) store_out([&](int64_t at, float v) { static_cast<float*>(P.out)[at] = v; });
+  else store_out([&](int64_t at, float v) { store_as(P.out, at, P.odt, v); });
 }
 // ---------------------------------------------------------------------------
 // key-parallel output pass (bf16 operands, head_dim 64: the training forward
@@ -680,7 +687,7 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_out(FwdParams P) {
 // normalises.  With 16 waves (512 keys) a CU holds one workgroup (148 KB of
 // LDS) and there are half the partials of 8 waves.
 
-template <int D, int KW>
+template <int D, int KW, bool FLAT = true>
 __global__ __launch_bounds__(64 * KW, 16 / KW) void fwd_keyout(FwdParams P, __bf16* __restrict__ op,
                                                                float* __restrict__ rp, int64_t ntiles) {
   static_assert(D == 64, "the key-parallel output pass is built for head_dim 64");
@@ -717,9 +724,9 @@ __global__ __launch_bounds__(64 * KW, 16 / KW) void fwd_keyout(FwdParams P, __bf
   const bool key_ok = key < T;
   const bool active = static_cast<int64_t>(kb) * kTileK < T;
 
-  const CT* qs = static_cast<const CT*>(P.q) + slice * P.q_sn;
+  const CT* qs = static_cast<const CT*>(P.q) + P.qv.slice(P.s0 + slice);
   RowFrag<CT, D> kf;
-  if (key_ok) load_row_frag<CT, D>(kf, static_cast<const CT*>(P.k) + slice * P.k_sn + key * D + h * (D / 2));
+  if (key_ok) load_row_frag<CT, D>(kf, static_cast<const CT*>(P.k) + P.kv.slice(P.s0 + slice) + key * P.kv.sr + h * (D / 2));
   else zero_row_frag<CT, D>(kf);
   // the parked V fragments: fragment (d quarter u, key step w, lane) holds
   // V[32 (kb0 + w) + 8 (lane >> 4) + t][16 u + (lane & 15)], t = 0..7, zero
@@ -734,11 +741,15 @@ __global__ __launch_bounds__(64 * KW, 16 / KW) void fwd_keyout(FwdParams P, __bf
   static_assert(kVChunks == D / 16, "one register set serves both parking forms");
   if (P.v != nullptr) {
     const int64_t first = static_cast<int64_t>(kb0) * kTileK;            // the group's first key
-    const CT* vs = static_cast<const CT*>(P.v) + slice * P.v_sn + first * D;
-    const auto rs = make_rsrc(vs, (T - first) * D * static_cast<int64_t>(sizeof(CT)));
+    const CT* vs = static_cast<const CT*>(P.v) + P.vv.slice(P.s0 + slice) + first * P.vv.sr;
+    const auto rs = make_rsrc(vs, rows_bytes<CT, D>(T - first, P.vv.sr));
+    const uint32_t ldb = static_cast<uint32_t>(P.vv.sr) * static_cast<uint32_t>(sizeof(CT));
 #pragma unroll
     for (int c = 0; c < kVChunks; ++c)
-      vfr[c] = buffer_load16<bf16x8>(rs, static_cast<uint32_t>((threadIdx.x + c * KG::kThreads) * 16), 0);
+      {
+      const uint32_t i = threadIdx.x + static_cast<uint32_t>(c) * KG::kThreads;
+      vfr[c] = buffer_load16<bf16x8>(rs, (i / (D / 8)) * ldb + (i % (D / 8)) * 16u, 0);
+    }
   } else {
     const CT* vts = static_cast<const CT*>(P.vt) + slice * P.t_sn;
     const int64_t first = static_cast<int64_t>(kb0) * kTileK * D;
@@ -767,12 +778,13 @@ __global__ __launch_bounds__(64 * KW, 16 / KW) void fwd_keyout(FwdParams P, __bf
   float lz = 0.f;
   const float* rmax = P.rmax + slice * P.C;
   const float* rden = P.rden + slice * P.C;
+  const int qld = FLAT ? D : static_cast<int>(P.qv.sr);
+  const uint32_t qoff = FLAT ? static_cast<uint32_t>(c256 * 16)
+                             : static_cast<uint32_t>((c256 / (D / 8)) * qld * 2 + (c256 % (D / 8)) * 16);
   auto fetch = [&](int rt) {
     const int64_t row0 = static_cast<int64_t>(rt) * kTileQ;
-    const int64_t rows = min(max(C - row0, int64_t{0}), int64_t{kTileQ});
     if (stager)
-      rr = buffer_load16<bf16x8>(make_rsrc(qs + row0 * D, rows * D * static_cast<int64_t>(sizeof(CT))),
-                                 static_cast<uint32_t>(c256 * 16), 0);
+      rr = buffer_load16<bf16x8>(tile_rsrc<CT, D>(qs, rt * kTileQ, static_cast<int>(C), qld), qoff, 0);
     if (threadIdx.x < kTileQ) {
       const int64_t r = row0 + threadIdx.x;
       lz = r < C ? rmax[r] + __log2f(rden[r]) : INFINITY;
@@ -938,9 +950,11 @@ __global__ __launch_bounds__(64 * KW, 16 / KW) void fwd_keyout(FwdParams P, __bf
 template <int D, int KW>
 __global__ __launch_bounds__(kThreads) void fwd_out_reduce(const __bf16* __restrict__ op,
                                                            const float* __restrict__ rp, int64_t ntiles,
-                                                           int64_t T, int64_t Tk, float* __restrict__ out,
-                                                           int64_t o_sn, float* __restrict__ ssum, int64_t slice0) {
-  // T: the chunk's rows; Tk: keys (the chunk starts at row Tk - T)
+                                                           int64_t T, int64_t Tk, void* __restrict__ out,
+                                                           RowsView ov, int odt, int64_t out0,
+                                                           float* __restrict__ ssum, int64_t slice0) {
+  // T: the chunk's rows; Tk: keys (the chunk starts at row Tk - T); out0: the
+  // output's slice of this batch's first slice
   static_assert(D * kTileQ == 8 * kThreads, "one 16-byte chunk of the partial tile per thread");
   __shared__ float sum_s[D][kTileQ + 1];
   __shared__ float s_s[kTileQ];
@@ -995,15 +1009,10 @@ __global__ __launch_bounds__(kThreads) void fwd_out_reduce(const __bf16* __restr
   const int64_t grow = static_cast<int64_t>(tq) * kTileQ + row;
   if (grow < T) {
     const float inv = 1.f / (s_s[row] + kEps);
-    floatx4 a, b;
+    float v[8];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      a[e] = sum_s[d8 + e][row] * inv;
-      b[e] = sum_s[d8 + 4 + e][row] * inv;
-    }
-    floatx4* o = reinterpret_cast<floatx4*>(out + slice * o_sn + grow * D + d8);
-    o[0] = a;
-    o[1] = b;
+    for (int e = 0; e < 8; ++e) v[e] = sum_s[d8 + e][row] * inv;
+    store8_as(out, ov.slice(out0 + slice) + grow * ov.sr + d8, odt, v);
   }
 }
 
@@ -1098,25 +1107,25 @@ int launch_forward(const ForwardArgs& a) {
   slice_batches(a.n, [&](int64_t s0, unsigned ns) {
     PrepJobs kv{};
     unsigned nkv = 0;
-    if (!v_rows) kv.job[nkv++] = PrepJob{a.v, a.kv_sn, nullptr, 0, vt, nullptr};
-    if (convert || kt != nullptr) kv.job[nkv++] = PrepJob{a.k, a.kv_sn, kc, a.Tk * D, kt, nullptr};
+    if (!v_rows) kv.job[nkv++] = PrepJob{a.v, a.vv, nullptr, 0, vt, nullptr};
+    if (convert || kt != nullptr) kv.job[nkv++] = PrepJob{a.k, a.kv, kc, a.Tk * D, kt, nullptr};
     if (nkv > 0)
       DIL_TIMED("prep", st, (prep_kernel<CT, D><<<dim3(ktiles, ns, nkv), kThreads, 0, st>>>(
                                 kv, a.dtype, a.Tk, D * tk_pad, tk_pad, s0)));
     if (convert) {
       PrepJobs qj{};
-      qj.job[0] = PrepJob{a.q, a.q_sn, qc, a.C * D, nullptr, nullptr};
+      qj.job[0] = PrepJob{a.q, a.qv, qc, a.C * D, nullptr, nullptr};
       DIL_TIMED("prep", st, (prep_kernel<CT, D><<<dim3(qtiles, ns, 1), kThreads, 0, st>>>(qj, a.dtype, a.C, 0, 0, s0)));
     }
   });
 
   FwdParams P{};
   P.q = convert ? static_cast<const void*>(qc) : a.q;
-  P.q_sn = convert ? a.C * D : a.q_sn;
+  P.qv = convert ? flat_rows(a.C * D, D) : a.qv;
   P.k = convert ? static_cast<const void*>(kc) : a.k;
-  P.k_sn = convert ? a.Tk * D : a.kv_sn;
+  P.kv = convert ? flat_rows(a.Tk * D, D) : a.kv;
   P.v = v_rows ? a.v : nullptr;
-  P.v_sn = a.kv_sn;
+  P.vv = a.vv;
   P.vt = vt;
   P.kt = kt;
   P.t_sn = D * tk_pad;
@@ -1131,7 +1140,8 @@ int launch_forward(const ForwardArgs& a) {
   P.scale = 1.f / sqrtf(static_cast<float>(D));
   P.c = kLog2e * P.scale;
   P.out = a.out;
-  P.o_sn = a.o_sn;
+  P.ov = a.ov;
+  P.odt = a.out_dtype;
   P.rmax = a.rmax;
   P.rden = a.rden;
   P.ssum = a.ssum;
@@ -1145,10 +1155,13 @@ int launch_forward(const ForwardArgs& a) {
   P.lshift = log2f(a.var.shift);
 
   P.n = a.n;
+  const bool flat = P.qv.sr == D && P.kv.sr == D && P.vv.sr == D;
   P.groups = static_cast<int>((a.C + 4 * kTileQ - 1) / (4 * kTileQ));
   const dim3 grid(static_cast<unsigned>(xcd_grid(P.groups * a.n)));
-  if (a.pk) DIL_TIMED("fwd_stats", st, (fwd_stats<CT, D, true, BID><<<grid, kThreads, 0, st>>>(P)));
-  else DIL_TIMED("fwd_stats", st, (fwd_stats<CT, D, false, BID><<<grid, kThreads, 0, st>>>(P)));
+  const int strided = with_rows<is_production<BID, SHARE>() && D <= 128>(flat, [&](auto flat_tag) -> int {
+  constexpr bool kFlat = decltype(flat_tag)::value;
+  if (a.pk) DIL_TIMED("fwd_stats", st, (fwd_stats<CT, D, true, BID, kFlat><<<grid, kThreads, 0, st>>>(P)));
+  else DIL_TIMED("fwd_stats", st, (fwd_stats<CT, D, false, BID, kFlat><<<grid, kThreads, 0, st>>>(P)));
   if constexpr (kKeyPassBuilt) {
     if (key_pass) {
       // one key pass forms the checkpoints, the totals and the share V
@@ -1173,9 +1186,7 @@ int launch_forward(const ForwardArgs& a) {
         const int64_t nbat = min(batch, a.n - b0);
         FwdParams B = P;
         B.n = nbat;
-        B.q = static_cast<const CT*>(P.q) + b0 * P.q_sn;
-        B.k = static_cast<const CT*>(P.k) + b0 * P.k_sn;
-        if (P.v != nullptr) B.v = static_cast<const CT*>(P.v) + b0 * P.v_sn;
+        B.s0 = b0;
         B.vt = static_cast<const CT*>(P.vt) + b0 * P.t_sn;
         B.rmax = P.rmax + b0 * P.C;
         B.rden = P.rden + b0 * P.C;
@@ -1183,13 +1194,12 @@ int launch_forward(const ForwardArgs& a) {
         if (P.demand_in != nullptr) B.demand_in = P.demand_in + b0 * P.din_sn;
         B.total = P.total + b0 * P.tot_sn;
         const dim3 gko(static_cast<unsigned>(xcd_grid(static_cast<int64_t>(B.kgroups) * nbat)));
-        DIL_TIMED("fwd_keyout", st, (fwd_keyout<D, KW><<<gko, KG::kThreads, 0, st>>>(B, op, rp, ntiles)));
-        float* out_b = a.out + b0 * a.o_sn;
+        DIL_TIMED("fwd_keyout", st, (fwd_keyout<D, KW, kFlat><<<gko, KG::kThreads, 0, st>>>(B, op, rp, ntiles)));
         float* ssum_b = a.ssum + b0 * a.C;
         slice_batches(nbat, [&](int64_t s0, unsigned ns) {
           DIL_TIMED("fwd_out_reduce", st,
-                    (fwd_out_reduce<D, KW><<<dim3(nq, ns), kThreads, 0, st>>>(op, rp, ntiles, a.C, a.Tk, out_b,
-                                                                             a.o_sn, ssum_b, s0)));
+                    (fwd_out_reduce<D, KW><<<dim3(nq, ns), kThreads, 0, st>>>(
+                        op, rp, ntiles, a.C, a.Tk, a.out, a.ov, a.out_dtype, b0, ssum_b, s0)));
         });
       }
       return static_cast<int>(hipGetLastError());
@@ -1197,10 +1207,12 @@ int launch_forward(const ForwardArgs& a) {
   }
   P.kgroups = static_cast<int>((a.Tk + 4 * kTileK - 1) / (4 * kTileK));
   DIL_TIMED("fwd_demand", st,
-            (fwd_demand<CT, D, BID><<<dim3(static_cast<unsigned>(xcd_grid(static_cast<int64_t>(P.kgroups) * a.n))),
+            (fwd_demand<CT, D, BID, kFlat><<<dim3(static_cast<unsigned>(xcd_grid(static_cast<int64_t>(P.kgroups) * a.n))),
                                       kThreads, 0, st>>>(P)));
-  DIL_TIMED("fwd_out", st, (fwd_out<CT, D, BID, SHARE><<<grid, kThreads, 0, st>>>(P)));
+  DIL_TIMED("fwd_out", st, (fwd_out<CT, D, BID, SHARE, kFlat><<<grid, kThreads, 0, st>>>(P)));
   return static_cast<int>(hipGetLastError());
+  });
+  return strided;
 }
 
 }  // namespace

@@ -5,6 +5,8 @@
 #include <stdint.h>
 #include <stdlib.h>
 
+#include <type_traits>
+
 namespace dil {
 
 // Negative status codes (positive values are hipError_t).  Mirrored by
@@ -27,6 +29,46 @@ struct Variant {
   float shift = 1.f;
 };
 int check_variant(const Variant& v, int head_dim);
+
+// Where the rows of the slices (batch b, head h, slice b * heads + h) of a
+// (B, H, T, D) tensor start: strides in elements, head dims contiguous.  The
+// kernels read q, k, v and dout and write the gradients and the outputs through
+// it, so views of a fused projection need no contiguous copies.  `magic` =
+// ceil(2^32 / heads) gives b by one multiplication on the scalar unit (exact for
+// slices * heads < 2^32, which dil_api.hip checks): a division costs about 1 us
+// at the start of every workgroup.  Slices at equal steps have heads = 1 and
+// magic = 0, so b = 0 and h = the slice.
+struct RowsView {
+  uint32_t heads, magic;
+  int64_t sb, sh, sr;
+#if defined(__HIPCC__)
+  __host__ __device__
+#endif
+  int64_t slice(int64_t s) const {
+    uint32_t i = static_cast<uint32_t>(s);
+#if defined(__HIP_DEVICE_COMPILE__)
+    // the slice is the same in every lane (a workgroup works on one slice):
+    // stated so, the offset and the row pointers stay in scalar registers
+    i = __builtin_amdgcn_readfirstlane(i);
+#endif
+    const uint32_t b = static_cast<uint32_t>((static_cast<uint64_t>(i) * magic) >> 32);
+    return static_cast<int64_t>(b) * sb + static_cast<int64_t>(i - b * heads) * sh;
+  }
+};
+inline RowsView flat_rows(int64_t slice_stride, int64_t row_stride) {
+  return RowsView{1, 0, 0, slice_stride, row_stride};
+}
+
+// f(std::true_type) when the rows of q, k and v lie head_dim elements apart,
+// f(std::false_type) for strided rows: two forms of the kernels.  The ablation
+// variants and head_dim 256 are built in the flat form only (kErrShape for
+// strided rows; the Python layer makes contiguous copies for them).
+template <bool STRIDED_BUILT, typename F>
+inline int with_rows(bool flat, F&& f) {
+  if (flat) return f(std::true_type{});
+  if constexpr (STRIDED_BUILT) return f(std::false_type{});
+  else return kErrShape;
+}
 
 inline size_t align_up(size_t bytes) { return (bytes + 255) & ~static_cast<size_t>(255); }
 
@@ -89,15 +131,17 @@ int decode_step(const DecodeArgs& a);
 // Forward over query rows [q0, q0 + C) against keys [0, Tk), Tk = q0 + C.
 // Plain forward: q0 = 0, C = Tk = T.  Chunked prefill: q0 = chunk start.
 struct ForwardArgs {
-  const void* q;         // (n, C, D) rows, slice stride q_sn
-  int64_t q_sn;
-  const void* k;         // (n, >= Tk, D), slice stride kv_sn
+  const void* q;         // C rows per slice
+  RowsView qv;
+  const void* k;         // >= Tk rows per slice
+  RowsView kv;
   const void* v;
-  int64_t kv_sn;
+  RowsView vv;
   int64_t n, C, Tk, q0;
   int head_dim, dtype, prec;   // precision code: 0 fp32, 1 split (tf32), 2 bf16 MFMA operands
-  float* out;            // (n, C, D) fp32, slice stride o_sn
-  int64_t o_sn;
+  void* out;             // C rows per slice, in out_dtype
+  RowsView ov;
+  int out_dtype;
   float* rmax;           // (n, C) fp32 (log2-domain row max of the scaled affinities)
   float* rden;           // (n, C) fp32 (sum of 2^(a - rmax))
   float* ssum;           // (n, C) fp32 (row sum of shares)
@@ -134,10 +178,12 @@ bool forward_takes_key_pass(int64_t C, int64_t Tk, int64_t q0, int head_dim, int
 int forward(const ForwardArgs& a);
 
 struct BackwardArgs {
-  const void* q;         // (n, T, D) each, contiguous slices of T*D
+  const void* q;         // T rows per slice
   const void* k;
   const void* v;
-  const void* dout;      // (n, T, D) in dout_dtype
+  RowsView qv, kv, vv;
+  const void* dout;      // T rows per slice, in dout_dtype
+  RowsView dov;
   const float* out;      // (n, T, D) fp32 forward output
   const float* rmax;     // (n, T)
   const float* rden;
@@ -145,9 +191,10 @@ struct BackwardArgs {
   const float* carry;    // (n, ceil(T/32), T)
   const float* pk;       // (n, T, D)
   Variant var;
-  void* dq;              // (n, T, D) each in grad_dtype
+  void* dq;              // T rows per slice, in grad_dtype
   void* dk;
   void* dv;
+  RowsView gqv, gkv, gvv;
   int64_t n, T;
   int head_dim, dtype, dout_dtype, grad_dtype, prec;   // prec as in ForwardArgs
   void* workspace;

@@ -4,6 +4,7 @@
 #pragma once
 
 #include "dil_common.hpp"
+#include "dil_internal.hpp"
 
 namespace dil {
 
@@ -69,13 +70,13 @@ __device__ __forceinline__ void load8(const CT* src, float (&v)[8]) {
   }
 }
 
-// One operand preparation: rows of `src` (slice stride src_sn) in the compute
+// One operand preparation: the rows of `src` (layout `sv`) in the compute
 // type, optionally scaled per row by rscale[(slice, row)] (in fp32, before the
 // rounding): a row-major copy into dst (slice stride dst_sn) and/or a
 // tile-major transposed copy into dst_t.  Null outputs are skipped.
 struct PrepJob {
   const void* src;
-  int64_t src_sn;
+  RowsView sv;
   void* dst;
   int64_t dst_sn;
   void* dst_t;
@@ -98,19 +99,20 @@ __global__ __launch_bounds__(kThreads) void prep_kernel(PrepJobs jobs, int dt, i
                                                         int64_t rows_pad, int64_t slice0) {
   const PrepJob& job = jobs.job[blockIdx.z];
   const void* __restrict__ src = job.src;
-  const int64_t src_sn = job.src_sn, dst_sn = job.dst_sn;
+  const int64_t dst_sn = job.dst_sn;
   CT* __restrict__ dst = static_cast<CT*>(job.dst);
   CT* __restrict__ dst_t = static_cast<CT*>(job.dst_t);
   const float* __restrict__ rscale = job.rscale;
   __shared__ float tile[64][D + 1];
   const int64_t slice = slice0 + blockIdx.y;
   const int64_t r0 = static_cast<int64_t>(blockIdx.x) * 64;
+  const int64_t src0 = job.sv.slice(slice), ld = job.sv.sr;
   constexpr int kVecPerRow = D / 8;
   for (int idx = threadIdx.x; idx < 64 * kVecPerRow; idx += kThreads) {
     const int r = idx / kVecPerRow, c8 = (idx % kVecPerRow) * 8;
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (r0 + r < rows) {
-      load8_f32(src, slice * src_sn + (r0 + r) * D + c8, dt, v);
+      load8_f32(src, src0 + (r0 + r) * ld + c8, dt, v);
       if (rscale != nullptr) {
         const float f = rscale[slice * rows + r0 + r];
 #pragma unroll
@@ -280,6 +282,29 @@ __device__ __forceinline__ V buffer_load16(__amdgpu_buffer_rsrc_t r, uint32_t vo
 __device__ __forceinline__ float buffer_load_f32(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
 }
+// Bytes from the first of `rows` rows (ld >= D elements apart) to the end of
+// the last one: a resource of this size covers exactly those rows, so a chunk
+// of a later row reads as zeros.
+template <typename CT, int D>
+__device__ __forceinline__ int64_t rows_bytes(int64_t rows, int64_t ld) {
+  return rows > 0 ? ((rows - 1) * ld + D) * static_cast<int64_t>(sizeof(CT)) : 0;
+}
+// The resource over rows [row0, row0 + 32) of a slice of `rows` rows, as far
+// as they exist.  In 32 bits throughout (slices hold fewer than 2^31 rows, ld is
+// below 2^20): 64-bit comparisons would leave the scalar unit.
+template <typename CT, int D>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const CT* base, int row0, int rows, int ld) {
+  const int r0 = __builtin_amdgcn_readfirstlane(row0), l = __builtin_amdgcn_readfirstlane(ld);
+  // min(rows left, 32) rows: (n - 1) l + D elements, none when n <= 0 (l >= D)
+  const int n = max(min(__builtin_amdgcn_readfirstlane(rows) - r0, kTileK), 0);
+  const int bytes = max(n * l - (l - D), 0) * static_cast<int>(sizeof(CT));
+  const uint64_t a = reinterpret_cast<uint64_t>(base) +
+                     static_cast<uint64_t>(static_cast<uint32_t>(r0)) * (static_cast<uint32_t>(l) * static_cast<uint32_t>(sizeof(CT)));
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(a));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(a >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>((static_cast<uint64_t>(hi) << 32) | lo), 0, bytes,
+                                           0x00020000);
+}
 // Loads of a split reduction's partials, which are read exactly once: the
 // non-temporal hint streams them past the caches instead of evicting reused
 // data (measured 11% faster on the partial reductions).
@@ -324,7 +349,8 @@ enum LoadMode { kLoadBuffer = 0, kLoadClamp = 1, kLoadSkip = 2 };
 // query-split order (row r at slot qs_slot(r)): lanes that read rows qsig(l)
 // then read consecutive slots, which keeps their 16-byte LDS reads free of
 // bank conflicts (rows r and r + 16 of the natural order share banks).
-template <typename CT, int D, bool QS = false, int MODE = kLoadBuffer>
+// FLAT: the rows lie D elements apart (load's ld is not read); else ld apart.
+template <typename CT, int D, bool QS = false, int MODE = kLoadBuffer, bool FLAT = true>
 struct KTileLoader {
   using T = Tiles<CT, D>;
   using V = typename Vec16<CT>::type;
@@ -332,29 +358,47 @@ struct KTileLoader {
   static constexpr int kPerRow = D / T::kChunk;
   V r[kPer];
   int nrows;                                        // rows inside the slice (clamp form)
-  __device__ void load(const CT* base, int64_t key0, int64_t nkeys) {
-    if constexpr (MODE == kLoadBuffer) {
+  // ld: elements from one row to the next (>= D)
+  __device__ void load(const CT* base, int64_t key0, int64_t nkeys, int64_t ld) {
+    if constexpr (MODE == kLoadBuffer && FLAT) {
       const int64_t rows = min(max(nkeys - key0, int64_t{0}), int64_t{kTileK});
       const auto rs = make_rsrc(base + key0 * D, rows * D * static_cast<int64_t>(sizeof(CT)));
 #pragma unroll
       for (int u = 0; u < kPer; ++u)   // chunks idx >= kKChunks lie past the tile: zeros, never stored
         r[u] = buffer_load16<V>(rs, static_cast<uint32_t>((threadIdx.x + u * kThreads) * 16), 0);
+    } else if constexpr (MODE == kLoadBuffer) {
+      const auto rs = tile_rsrc<CT, D>(base, static_cast<int>(key0), static_cast<int>(nkeys), static_cast<int>(ld));
+      static_assert(kThreads % kPerRow == 0, "a thread's chunks lie in one column of chunks");
+      const uint32_t lds = static_cast<uint32_t>(ld) * static_cast<uint32_t>(sizeof(CT));
+      const uint32_t off = (threadIdx.x / kPerRow) * lds + (threadIdx.x % kPerRow) * 16u;
+#pragma unroll
+      for (int u = 0; u < kPer; ++u)   // chunks idx >= kKChunks lie past the tile: zeros, never stored
+        r[u] = buffer_load16<V>(rs, off + static_cast<uint32_t>(u * (kThreads / kPerRow)) * lds, 0);
     } else {
       // slices hold fewer than 2^31 rows
       const int k0 = static_cast<int>(key0), last = static_cast<int>(nkeys) - 1;
       nrows = min(max(last + 1 - k0, 0), kTileK);
+      // strided clamp form: the tile's first row (the last one, for a tile past
+      // the end) in 64 bits, the lanes' rows relative to it in 32
+      [[maybe_unused]] const int c0 = min(k0, last), l = static_cast<int>(ld);
+      [[maybe_unused]] const int top = min(last - c0, kTileK - 1) * l;
+      [[maybe_unused]] const CT* tile = base + static_cast<int64_t>(c0) * l;
 #pragma unroll
       for (int u = 0; u < kPer; ++u) {
-        if constexpr (MODE == kLoadClamp) {
+        if constexpr (MODE == kLoadClamp && FLAT) {
           const int idx = min(static_cast<int>(threadIdx.x) + u * kThreads, T::kKChunks - 1);
           const int row = min(k0 + idx / kPerRow, last);
           r[u] = *reinterpret_cast<const V*>(base + static_cast<int64_t>(row) * D + (idx % kPerRow) * T::kChunk);
+        } else if constexpr (MODE == kLoadClamp) {
+          const int idx = min(static_cast<int>(threadIdx.x) + u * kThreads, T::kKChunks - 1);
+          const uint32_t off = static_cast<uint32_t>(min((idx / kPerRow) * l, top) + (idx % kPerRow) * T::kChunk);
+          r[u] = *reinterpret_cast<const V*>(tile + off);
         } else {
           const int idx = threadIdx.x + u * kThreads;
           const int row = idx / kPerRow;
           r[u] = V{};
           if (idx < T::kKChunks && row < nrows)
-            r[u] = *reinterpret_cast<const V*>(base + (key0 + row) * D + (idx % kPerRow) * T::kChunk);
+            r[u] = *reinterpret_cast<const V*>(base + (key0 + row) * (FLAT ? D : ld) + (idx % kPerRow) * T::kChunk);
         }
       }
     }

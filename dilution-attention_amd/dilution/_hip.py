@@ -19,6 +19,16 @@ _c_int64 = ctypes.c_int64
 _c_int = ctypes.c_int
 _vp = ctypes.c_void_p
 
+
+class Rows(ctypes.Structure):
+    """``dil_rows``: where the rows of a (B, H, T, D) tensor start."""
+
+    _fields_ = [("data", _vp), ("batch_stride", _c_int64), ("head_stride", _c_int64),
+                ("row_stride", _c_int64)]
+
+
+_rows_p = ctypes.POINTER(Rows)
+
 # name -> (restype, argtypes); must match include/dilution_hip.h
 SIGNATURES = {
     "dil_abi_version": (_c_int, []),
@@ -41,6 +51,16 @@ SIGNATURES = {
                                       _c_int64, _c_int, _c_int, _c_int, _c_int, _c_int,
                                       _c_int, _c_int, ctypes.c_float,
                                       _vp, _vp, _vp, _vp, _c_int64, _vp]),
+    "dil_forward_rows": (_c_int, [_rows_p, _rows_p, _rows_p, _c_int64, _c_int64, _c_int64, _c_int, _c_int,
+                                  _c_int, _c_int, _c_int, ctypes.c_float,
+                                  _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_int64, _vp]),
+    "dil_backward_rows": (_c_int, [_rows_p, _rows_p, _rows_p, _rows_p, _vp, _vp, _vp, _vp, _vp, _vp,
+                                   _c_int64, _c_int64, _c_int64, _c_int, _c_int, _c_int, _c_int, _c_int,
+                                   _c_int, _c_int, ctypes.c_float, _rows_p, _rows_p, _rows_p, _vp,
+                                   _c_int64, _vp]),
+    "dil_prefill_rows": (_c_int, [_rows_p, _vp, _vp, _c_int64, _c_int64, _c_int64, _c_int64, _c_int64,
+                                  _c_int, _c_int, _c_int, _vp, _rows_p, _c_int, _vp, _vp, _vp, _vp, _vp,
+                                  _c_int64, _vp]),
     "dil_decode_step_variant": (_c_int, [_vp, _vp, _vp, _vp, _vp, _c_int64, _c_int64, _c_int64,
                                          _c_int, _c_int, _c_int, _c_int, _c_int, ctypes.c_float,
                                          _vp, _c_int64, _vp]),

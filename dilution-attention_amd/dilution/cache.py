@@ -84,12 +84,13 @@ def begin_cache(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, capacity: int
         return y.to(q.dtype), cache
     if chunk < 1:
         raise ValueError("chunk must be positive")
-    outs = []
+    # every chunk writes its rows of y, in q's type
+    y = torch.empty(q.shape, device=q.device, dtype=q.dtype)
     for start in range(0, seq, chunk):
         stop = min(start + chunk, seq)
-        outs.append(kernels.dilution_prefill_chunk(q[:, :, start:stop], cache["k"], cache["v"],
-                                                   cache["committed"], start, dot_precision=prec))
-    return torch.cat(outs, dim=2).to(q.dtype), cache
+        kernels.dilution_prefill_chunk(q[:, :, start:stop], cache["k"], cache["v"], cache["committed"], start,
+                                       dot_precision=prec, _out=y[:, :, start:stop])
+    return y, cache
 
 
 def step_cache(q1: torch.Tensor, k1: torch.Tensor, v1: torch.Tensor, cache: dict, **bid_kw) -> torch.Tensor:

@@ -156,6 +156,69 @@ def _rows(x: torch.Tensor, n: int, t: int, d: int, dtype: torch.dtype) -> torch.
     return x.reshape(n, t, d).to(dtype).contiguous()
 
 
+def _strided_rows(x: torch.Tensor) -> bool:
+    """Whether the kernels read (or write) this (B, H, T, D) tensor where it
+    lies (the layout rules of ``dil_rows``): contiguous head dims, rows and
+    slices at 16-byte steps, the row stride from head_dim to 2^20 elements.
+    Rows that are apart also have to lie within 2^31 bytes, which the one-pass
+    backward's 32-bit offsets cover."""
+    batch, heads, seq, head_dim = x.shape
+    sb, sh, st, sd = x.stride()
+    es = x.element_size()
+    lane = 16 // es
+    return (sd == 1 and head_dim <= st < (1 << 20) and st % lane == 0
+            and (batch == 1 or sb % lane == 0) and (heads == 1 or sh % lane == 0)
+            and (st == head_dim or seq * st * es < (1 << 31)) and x.data_ptr() % 16 == 0)
+
+
+def _operand(x: torch.Tensor, dtype: torch.dtype, flat: bool = False) -> torch.Tensor:
+    """x (B, H, T, D) in `dtype` as the kernels can read it: x itself when
+    its type and layout allow (views of a fused projection do), else a
+    contiguous copy.  `flat`: rows head_dim apart."""
+    x = x.to(dtype)
+    if flat:
+        x = x.contiguous()
+    return x if _strided_rows(x) else x.clone(memory_format=torch.contiguous_format)
+
+
+def _slice_dims(batch: int, heads: int) -> tuple[int, int]:
+    """(batch, heads) as the kernels count slices: as they are within
+    ``dil_rows``' limits, else every slice a batch of its own."""
+    if heads < 1 << 16 and batch * heads * heads < 1 << 32:
+        return batch, heads
+    return batch * heads, 1
+
+
+def _sliced(x: torch.Tensor, dims: tuple[int, int]) -> torch.Tensor:
+    """x (B, H, T, D) with its slices counted as `dims`."""
+    if x.shape[:2] == dims:
+        return x
+    return x.contiguous().view(*dims, *x.shape[2:])
+
+
+def _flat_only(variant: tuple, head_dim: int) -> bool:
+    """The calls whose kernels are built for rows head_dim apart only: the
+    ablation variants, and head_dim 256 (no registers for a row stride)."""
+    return head_dim > 128 or tuple(variant) != _PRODUCTION
+
+
+def _row_ref(x: torch.Tensor):
+    """``dil_rows`` of a (B, H, T, D) tensor that ``_strided_rows`` accepts."""
+    sb, sh, st, _ = x.stride()
+    return _hip.Rows(x.data_ptr(), sb, sh, st)
+
+
+def _empty_as(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """A new (B, H, T, D) tensor in `dtype` whose memory order follows x:
+    (B, T, H, D) when x's rows are stepped over heads first (the views of a
+    (B, T, H * D) projection), so that its view back to (B, T, H * D) needs no
+    copy; else contiguous."""
+    batch, heads, seq, head_dim = x.shape
+    if heads > 1 and seq > 1 and x.stride(1) < x.stride(2):
+        return torch.empty(batch, seq, heads, head_dim, device=x.device, dtype=dtype).transpose(1, 2)
+    return torch.empty(batch, heads, seq, head_dim, device=x.device, dtype=dtype)
+
+
 def _stream(dev: torch.device) -> int:
     """The caller's current stream on the inputs' device; launches go there.
     (The raw handle, without building a torch Stream object: a decode step
@@ -226,7 +289,7 @@ def dilution_attention_forward(
     lib = _hip.lib()
     n = batch * heads
     dt = _common_dtype(q, k, v)
-    qf, kf, vf = (_rows(x, n, seq, head_dim, dt) for x in (q, k, v))
+    qf, kf, vf = (_operand(x, dt, _flat_only(_variant, head_dim)) for x in (q, k, v))
     dev = q.device
     nb = (seq + CHECKPOINT_ROWS - 1) // CHECKPOINT_ROWS
     f32 = dict(device=dev, dtype=torch.float32)
@@ -250,18 +313,17 @@ def dilution_attention_forward(
         carry = torch.empty(rows, nb, seq, **f32)
     ws_bytes = lib.dil_forward_workspace_bytes(rows, seq, head_dim, _DTYPES[dt], prec, int(_save_pk))
     ws = _workspace(ws_bytes, dev)
+    dims = _slice_dims(batch, heads) if rows >= n else (n, 1)   # (n, 1): groups of slices
+    qf, kf, vf = (_sliced(x, dims) for x in (qf, kf, vf))
     for a in range(0, n, rows):
         b = min(a + rows, n)
-        head = (qf[a:b].data_ptr(), kf[a:b].data_ptr(), vf[a:b].data_ptr(), b - a, seq, head_dim,
-                _DTYPES[dt], prec)
-        tail = (out[a:b].data_ptr(), rmax[a:b].data_ptr(), rden[a:b].data_ptr(),
-                ssum[a:b].data_ptr(), _ptr(carry), total[a:b].data_ptr(),
-                None if pk is None else pk[a:b].data_ptr(), ws.data_ptr(), ws.numel(), _stream(dev))
+        part = (qf, kf, vf) if rows >= n else tuple(x[a:b] for x in (qf, kf, vf))
         with _on(dev):
-            if tuple(_variant) == _PRODUCTION:
-                status = lib.dil_forward(*head, *tail)
-            else:
-                status = lib.dil_forward_variant(*head, *_variant, *tail)
+            status = lib.dil_forward_rows(
+                *(_row_ref(x) for x in part), *part[0].shape[:2], seq, head_dim, _DTYPES[dt], prec, *_variant,
+                out[a:b].data_ptr(), rmax[a:b].data_ptr(), rden[a:b].data_ptr(), ssum[a:b].data_ptr(),
+                _ptr(carry), total[a:b].data_ptr(), None if pk is None else pk[a:b].data_ptr(),
+                ws.data_ptr(), ws.numel(), _stream(dev))
         _hip.check(status, "dil_forward")
 
     result = out.reshape(batch, heads, seq, head_dim)
@@ -314,31 +376,24 @@ def _backward(saved, dout, dot_precision: str, variant: tuple):
     n = batch * heads
     prec = _precision_code(dot_precision)
     dt = _common_dtype(q, k, v)
-    qf, kf, vf = (_rows(x, n, seq, head_dim, dt) for x in (q, k, v))
+    qf, kf, vf = (_operand(x, dt, _flat_only(variant, head_dim)) for x in (q, k, v))
     ddt = dout.dtype if dout.dtype in _DTYPES else torch.float32
-    dof = _rows(dout, n, seq, head_dim, ddt)
-    of = out.reshape(n, seq, head_dim)
+    dof = _operand(dout.reshape(q.shape), ddt)
     dev = q.device
-    grads = []
-    gdt = dt
-    dq = torch.empty(n, seq, head_dim, device=dev, dtype=gdt)
-    dk = torch.empty_like(dq)
-    dv = torch.empty_like(dq)
+    dims = _slice_dims(batch, heads)
+    qf, kf, vf, dof = (_sliced(x, dims) for x in (qf, kf, vf, dof))
+    # the gradients in the memory order of their inputs
+    dq, dk, dv = (_sliced(_empty_as(x, dt), dims) for x in (q, k, v))
     ws = _workspace(lib.dil_backward_workspace_bytes(n, seq, head_dim, _DTYPES[dt], prec), dev)
-    head = (qf.data_ptr(), kf.data_ptr(), vf.data_ptr(), dof.data_ptr(), of.data_ptr(),
-            rmax.data_ptr(), rden.data_ptr(), ssum.data_ptr(), carry.data_ptr(), pk.data_ptr(),
-            n, seq, head_dim, _DTYPES[dt], _DTYPES[ddt], _DTYPES[gdt], prec)
-    tail = (dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), ws.numel(), _stream(dev))
     with _on(dev):
-        if tuple(variant) == _PRODUCTION:
-            status = lib.dil_backward(*head, *tail)
-        else:
-            status = lib.dil_backward_variant(*head, *variant, *tail)
+        status = lib.dil_backward_rows(
+            _row_ref(qf), _row_ref(kf), _row_ref(vf), _row_ref(dof), out.data_ptr(), rmax.data_ptr(),
+            rden.data_ptr(), ssum.data_ptr(), carry.data_ptr(), pk.data_ptr(), *dims, seq, head_dim,
+            _DTYPES[dt], _DTYPES[ddt], _DTYPES[dt], prec, *variant, _row_ref(dq), _row_ref(dk), _row_ref(dv),
+            ws.data_ptr(), ws.numel(), _stream(dev))
     _hip.check(status, "dil_backward")
-    shape4 = (batch, heads, seq, head_dim)
-    for g, ref in zip((dq, dk, dv), (q, k, v)):
-        grads.append(g.reshape(shape4).to(ref.dtype))
-    return tuple(grads)
+    return tuple(g.view(ref.shape).to(ref.dtype) if dims != ref.shape[:2] else g.to(ref.dtype)
+                 for g, ref in zip((dq, dk, dv), (q, k, v)))
 
 
 def dilution_attention(
@@ -380,6 +435,7 @@ def dilution_prefill_chunk(
     start: int,
     dot_precision: str = "bf16",
     return_aux: bool = False,
+    _out: torch.Tensor | None = None,
 ):
     """Rows [start, start + C) of the operator over the cached keys
     [0, start + C), carrying the fp32 demand vector across chunks.
@@ -391,7 +447,9 @@ def dilution_prefill_chunk(
     (entries beyond start + C are not touched).  Returns the chunk's outputs
     (B, H, C, D) fp32, and with return_aux the chunk's rmax/rden/ssum/carry.
     Chaining chunks reproduces ``dilution_attention_forward`` row for row and
-    its ``aux["committed_total"]``.
+    its ``aux["committed_total"]``.  ``_out`` (a (B, H, C, D) view that
+    ``_strided_rows`` accepts, any float dtype) takes the outputs in place of a
+    new fp32 tensor.
     """
     prec = _precision_code(dot_precision)
     capacity = _check_cache(q, k_cache, v_cache, committed)
@@ -408,11 +466,11 @@ def dilution_prefill_chunk(
     kf = k_cache.view(n, capacity, head_dim)
     vf = v_cache.view(n, capacity, head_dim)
     cf = committed.view(n, capacity)
-    qf = _rows(q, n, chunk, head_dim, dt)
+    qf = _operand(q, dt, _flat_only(_PRODUCTION, head_dim))
     dev = q.device
     nb = (chunk + CHECKPOINT_ROWS - 1) // CHECKPOINT_ROWS
     f32 = dict(device=dev, dtype=torch.float32)
-    out = torch.empty(n, chunk, head_dim, **f32)
+    out = torch.empty(batch, heads, chunk, head_dim, **f32) if _out is None else _out
     rmax = torch.empty(n, chunk, **f32)
     rden = torch.empty(n, chunk, **f32)
     ssum = torch.empty(n, chunk, **f32)
@@ -421,17 +479,19 @@ def dilution_prefill_chunk(
     if return_aux or not lib.dil_forward_key_pass(chunk, start, head_dim, _DTYPES[dt], prec):
         carry = torch.empty(n, nb, start + chunk, **f32)
     ws = _workspace(lib.dil_prefill_workspace_bytes(n, chunk, start, head_dim, _DTYPES[dt], prec), dev)
+    dims = _slice_dims(batch, heads)
+    qf = _sliced(qf, dims)
+    rows = out if dims == out.shape[:2] else out.view(*dims, chunk, head_dim)
     with _on(dev):
-        status = lib.dil_prefill_chunk(
-            qf.data_ptr(), kf.data_ptr(), vf.data_ptr(), n, chunk, start, capacity, head_dim,
-            _DTYPES[dt], prec, cf.data_ptr(), out.data_ptr(), rmax.data_ptr(), rden.data_ptr(),
-            ssum.data_ptr(), _ptr(carry), ws.data_ptr(), ws.numel(), _stream(dev))
+        status = lib.dil_prefill_rows(
+            _row_ref(qf), kf.data_ptr(), vf.data_ptr(), *dims, chunk, start, capacity, head_dim,
+            _DTYPES[dt], prec, cf.data_ptr(), _row_ref(rows), _DTYPES[out.dtype], rmax.data_ptr(),
+            rden.data_ptr(), ssum.data_ptr(), _ptr(carry), ws.data_ptr(), ws.numel(), _stream(dev))
     _hip.check(status, "dil_prefill_chunk")
-    result = out.reshape(batch, heads, chunk, head_dim)
     if return_aux:
-        return result, dict(rmax=rmax, rden=rden, ssum=ssum, carry=carry,
+        return out, dict(rmax=rmax, rden=rden, ssum=ssum, carry=carry,
                             bwd_block_m=CHECKPOINT_ROWS, dot_precision=dot_precision)
-    return result
+    return out
 
 
 # ---------------------------------------------------------------------------

@@ -55,6 +55,21 @@ int dil_abi_version(void);
 const char* dil_status_string(int status);
 
 /*
+ * The rows of a (B, H, T, head_dim) tensor in any order of its dimensions: row
+ * t of head h of batch b starts at data + b batch_stride + h head_stride +
+ * t row_stride elements, its head_dim elements contiguous.  The *_rows entry
+ * points below take their tensors so: the views that a fused q/k/v projection
+ * gives need no contiguous copies.  data is 16-byte aligned, the strides of
+ * dimensions longer than 1 and the row stride are multiples of 16 bytes, the
+ * row stride is at least head_dim and below 2^20, B H < 2^31 and B H H < 2^32
+ * with H < 2^16; anything else is an argument error (-4).
+ */
+typedef struct dil_rows {
+  const void* data;
+  int64_t batch_stride, head_stride, row_stride;
+} dil_rows;
+
+/*
  * Whether a dil_forward call (start = 0, chunk = seq) or a dil_prefill_chunk
  * call of this shape takes the key-parallel output pass: 1 or 0.  Its demand
  * checkpoints are an output only, so such a call may pass carry = NULL (an
@@ -237,6 +252,32 @@ int dil_decode_step_variant(const void* q1, const void* k_cache, const void* v_c
                             int64_t length, int head_dim, int dtype, int q_dtype, int bid,
                             int share, float shift, void* workspace, int64_t workspace_bytes,
                             void* stream);
+
+/*
+ * The forward, the backward and a prefill chunk on strided rows: arguments and
+ * results of dil_forward_variant, dil_backward_variant and dil_prefill_chunk
+ * with n = batch * heads, q, k, v, dout and the gradients as dil_rows (the
+ * forward's own outputs stay contiguous; the bid / share variants and
+ * head_dim 256 take q, k and v with row_stride == head_dim).  dil_prefill_rows also writes its
+ * output rows in `out_dtype` to any place, such as a chunk's rows of the whole
+ * prompt's output.  No reference counterpart: the reference makes contiguous
+ * copies (src/dilution/kernels.py:362-364).
+ */
+int dil_forward_rows(const dil_rows* q, const dil_rows* k, const dil_rows* v, int64_t batch, int64_t heads,
+                     int64_t seq, int head_dim, int dtype, int precision, int bid, int share, float shift,
+                     float* out, float* rmax, float* rden, float* ssum, float* carry, float* committed_total,
+                     float* pk, void* workspace, int64_t workspace_bytes, void* stream);
+int dil_backward_rows(const dil_rows* q, const dil_rows* k, const dil_rows* v, const dil_rows* dout,
+                      const float* out, const float* rmax, const float* rden, const float* ssum,
+                      const float* carry, const float* pk, int64_t batch, int64_t heads, int64_t seq,
+                      int head_dim, int dtype, int dout_dtype, int grad_dtype, int precision, int bid, int share,
+                      float shift, const dil_rows* dq, const dil_rows* dk, const dil_rows* dv, void* workspace,
+                      int64_t workspace_bytes, void* stream);
+int dil_prefill_rows(const dil_rows* q_chunk, const void* k_cache, const void* v_cache, int64_t batch,
+                     int64_t heads, int64_t chunk, int64_t start, int64_t capacity, int head_dim, int dtype,
+                     int precision, float* committed, const dil_rows* out, int out_dtype, float* rmax,
+                     float* rden, float* ssum, float* carry, void* workspace, int64_t workspace_bytes,
+                     void* stream);
 
 /*
  * Few-row projections of the LM's decode step.  No counterpart in the
