@@ -681,14 +681,28 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_out(FwdParams P) {
 //     same bf16 values that multiply V) are added on the VALU.
 // After the next tile's stash 8 waves form the tile's share V over the
 // group's keys, one 16 x 16 output block each (v_mfma_f32_16x16x32_bf16, V
-// parked in LDS), stored as one bf16 [64 x 32] partial (part_block_off) per (key group,
+// parked in LDS), stored as one [64 x 32] partial (part_block_off) per (key group,
 // tile) with the fp32 row sums beside it, compactly (ChunkGroups).
 // fwd_out_reduce sums the partials of every key group in a fixed order and
-// normalises.  With 16 waves (512 keys) a CU holds one workgroup (148 KB of
-// LDS) and there are half the partials of 8 waves.
+// normalises.
+//
+// Groups of 512 keys (16 waves, one workgroup per CU, bf16 partials) have the
+// fewest partials.  A walk takes its row tiles times ~2.05 us (the 16 waves'
+// instructions queue up on the CU's 4 SIMDs), so where such groups leave CUs idle
+// or their walks uneven, groups of 256 keys (8 waves: ~1.33 us per tile alone on a
+// CU, two workgroups fit one) finish sooner (keyout_waves): B2 H8 T4096 254 ->
+// 174 us, B3 H5 T1357 89 -> 67 us.  128 keys were no faster (1.23 us per tile: the
+// wave's own chain) and doubled the partials again.  The sums keep one order
+// whatever the groups, so the bits of a slice do not depend on the batch around
+// it: 128 keys in one MFMA chain, then (c0 + c1) + (c2 + c3) over a 512-key span in
+// fp32, rounded to bf16 there.  The 256-key groups store their part of that sum in
+// fp32 and fwd_out_reduce finishes it.
+
+// a group's partials: bf16 for a whole 512-key span, else fp32 parts of one
+template <int KW> using KoPart = std::conditional_t<KW == 16, __bf16, float>;
 
 template <int D, int KW, bool FLAT = true>
-__global__ __launch_bounds__(64 * KW, 16 / KW) void fwd_keyout(FwdParams P, __bf16* __restrict__ op,
+__global__ __launch_bounds__(64 * KW, 16 / KW) void fwd_keyout(FwdParams P, KoPart<KW>* __restrict__ op,
                                                                float* __restrict__ rp, int64_t ntiles) {
   static_assert(D == 64, "the key-parallel output pass is built for head_dim 64");
   static_assert(KW == 8 || KW == 16, "key groups of 256 or 512 keys");
@@ -865,31 +879,43 @@ __global__ __launch_bounds__(64 * KW, 16 / KW) void fwd_keyout(FwdParams P, __bf
   const int pw = wave - (KW - 8);
   const bool prod_wave = pw >= 0;                // wave-uniform
   const int rh = pw & 1, dq4 = (pw >> 1) & 3;
-  __bf16* op_s = op + slice * ntiles * (D * kTileQ);
+  KoPart<KW>* op_s = op + slice * ntiles * (D * kTileQ);
   float* rp_s = rp + slice * ntiles * kTileQ;
   const int64_t gbase = cg.base(kg) - rt0;
   auto product = [&](int rt, int buf) {
     if (rt < 0) return;
-    floatx4 acc = floatx4{};
     const CT* arow = sh_s[buf] + (16 * rh + (lane & 15)) * KG::kStride + 8 * (lane >> 4);
+    floatx4 c[KW / 4];
 #pragma unroll
-    for (int ks = 0; ks < KW; ++ks) {
-      const bf16x8 av = *reinterpret_cast<const bf16x8*>(arow + kTileK * ks);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, vpark[dq4][ks][lane], acc, 0, 0, 0);
+    for (int g = 0; g < KW / 4; ++g) {
+      c[g] = floatx4{};
+#pragma unroll
+      for (int ks = 4 * g; ks < 4 * g + 4; ++ks) {
+        const bf16x8 av = *reinterpret_cast<const bf16x8*>(arow + kTileK * ks);
+        c[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, vpark[dq4][ks][lane], c[g], 0, 0, 0);
+      }
     }
     // output: lane <-> head dim 16 dq4 + (lane & 15), register j <-> row 16 rh + 4 (lane >> 4) + j;
     // the partial tile is stored in 16 x 16 blocks (part_block_off), streamed past the caches
     const int64_t tile = gbase + rt;
-    const floatx2 a = {acc[0], acc[1]}, b = {acc[2], acc[3]};
-    const bf16x2 pa = __builtin_convertvector(a, bf16x2), pb = __builtin_convertvector(b, bf16x2);
-    const bf16x4 v = {pa[0], pa[1], pb[0], pb[1]};
-    __builtin_nontemporal_store(__builtin_bit_cast(floatx2, v),
-                                reinterpret_cast<floatx2*>(op_s + tile * (D * kTileQ) + part_block_off(dq4, rh, lane)));
+    KoPart<KW>* dst = op_s + tile * (D * kTileQ) + part_block_off(dq4, rh, lane);
+    if constexpr (KW == 16) {
+      const floatx4 acc = (c[0] + c[1]) + (c[2] + c[3]);
+      const floatx2 a = {acc[0], acc[1]}, b = {acc[2], acc[3]};
+      const bf16x2 pa = __builtin_convertvector(a, bf16x2), pb = __builtin_convertvector(b, bf16x2);
+      const bf16x4 v = {pa[0], pa[1], pb[0], pb[1]};
+      __builtin_nontemporal_store(__builtin_bit_cast(floatx2, v), reinterpret_cast<floatx2*>(dst));
+    } else {
+      __builtin_nontemporal_store(c[0] + c[1], reinterpret_cast<floatx4*>(dst));
+    }
     if (pw == 0 && lane < kTileQ) {
-      float s = 0.f;
+      float q[KW / 4];
 #pragma unroll
-      for (int w = 0; w < KW; ++w) s += rs_s[buf][w][lane];
-      __builtin_nontemporal_store(s, rp_s + tile * kTileQ + lane);
+      for (int g = 0; g < KW / 4; ++g)
+        q[g] = (rs_s[buf][4 * g][lane] + rs_s[buf][4 * g + 1][lane]) +
+               (rs_s[buf][4 * g + 2][lane] + rs_s[buf][4 * g + 3][lane]);
+      const float t = KW == 16 ? (q[0] + q[1]) + (q[KW / 4 - 2] + q[KW / 4 - 1]) : q[0] + q[1];
+      __builtin_nontemporal_store(t, rp_s + tile * kTileQ + lane);
     }
   };
 
@@ -948,7 +974,7 @@ __global__ __launch_bounds__(64 * KW, 16 / KW) void fwd_keyout(FwdParams P, __bf
 // groups first.  Thread t sums elements [8 t, 8 t + 8) of the partial tiles
 // (one head dim, 8 rows: part_dim / part_row).
 template <int D, int KW>
-__global__ __launch_bounds__(kThreads) void fwd_out_reduce(const __bf16* __restrict__ op,
+__global__ __launch_bounds__(kThreads) void fwd_out_reduce(const KoPart<KW>* __restrict__ op,
                                                            const float* __restrict__ rp, int64_t ntiles,
                                                            int64_t T, int64_t Tk, void* __restrict__ out,
                                                            RowsView ov, int odt, int64_t out0,
@@ -965,30 +991,46 @@ __global__ __launch_bounds__(kThreads) void fwd_out_reduce(const __bf16* __restr
   const int tq = nq - 1 - static_cast<int>(blockIdx.x);
   const int ng = static_cast<int>(min(KG::groups(Tk) - 1, cg.a + tq / KW)) + 1;
   const int t = threadIdx.x;
-  const __bf16* base = op + slice * ntiles * (D * kTileQ) + 8 * t;
+  const KoPart<KW>* base = op + slice * ntiles * (D * kTileQ) + 8 * t;
   auto tile_of = [&](int g) { return cg.base(g) + tq - cg.first(g); };
-  // groups in order, eight partial tiles in flight; threads 0-31 load the
-  // same groups' row sums beside them (both added in group order)
+  // spans of 512 keys in order, eight partial tiles in flight; threads 0-31 load
+  // the same groups' row sums beside them (both added in the same order).  A
+  // span of smaller groups adds up to its bf16 partial first; groups past the
+  // rows (keys after them) are zeros
   const bool srow = t < kTileQ;
   const float* gp = rp + slice * ntiles * kTileQ + (srow ? t : 0);
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   float s = 0.f;
+  constexpr int kSpan = 16 / KW;                 // groups per span
+  using Raw = std::conditional_t<KW == 16, bf16x8, floatx8>;
   for (int g = 0; g < ng; g += 8) {
-    bf16x8 v[8];
+    Raw v[8];
     float r[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
+      if constexpr (KW != 16) {
+        v[u] = Raw{};
+        r[u] = 0.f;
+      }
       if (g + u < ng) {
-        v[u] = load_once(base + tile_of(g + u) * (D * kTileQ));
+        if constexpr (KW == 16) v[u] = load_once(base + tile_of(g + u) * (D * kTileQ));
+        else v[u] = load8_once(base + tile_of(g + u) * (D * kTileQ));
         if (srow) r[u] = load_once(gp + tile_of(g + u) * kTileQ);
       }
     }
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < 8; u += kSpan) {
       if (g + u < ng) {
+        if constexpr (KW == 16) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] += static_cast<float>(v[u][e]);
-        if (srow) s += r[u];
+          for (int e = 0; e < 8; ++e) acc[e] += static_cast<float>(v[u][e]);
+          if (srow) s += r[u];
+        } else {
+          const floatx8 w = v[u] + v[u + 1];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[e] += static_cast<float>(static_cast<__bf16>(w[e]));
+          if (srow) s += r[u] + r[u + 1];
+        }
       }
     }
   }
@@ -1032,23 +1074,45 @@ __global__ __launch_bounds__(kThreads) void fwd_out_reduce(const __bf16* __restr
 constexpr int64_t kKeyoutBudgetBytes = int64_t{24} << 30;
 constexpr int kKeyoutWaves = 16;
 
-inline int64_t keyout_tiles(int64_t C, int64_t Tk) {
-  using KG = KeyGroups<kKeyoutWaves>;
-  const ChunkGroups<kKeyoutWaves> cg{(C + kTileQ - 1) / kTileQ, (Tk - C) / KG::kKeys};
-  return cg.base(KG::groups(Tk));
+template <int KW>
+inline int64_t keyout_tiles_of(int64_t C, int64_t Tk) {
+  const ChunkGroups<KW> cg{(C + kTileQ - 1) / kTileQ, (Tk - C) / KeyGroups<KW>::kKeys};
+  return cg.base(KeyGroups<KW>::groups(Tk));
 }
-inline int64_t keyout_partial_bytes(int64_t n, int64_t C, int64_t Tk, int D) {
-  return n * keyout_tiles(C, Tk) * (static_cast<int64_t>(D) * kTileQ * 2 + kTileQ * 4);
+inline int64_t keyout_tiles(int kw, int64_t C, int64_t Tk) {
+  return kw == 8 ? keyout_tiles_of<8>(C, Tk) : keyout_tiles_of<16>(C, Tk);
+}
+inline int64_t keyout_part_size(int kw) { return kw == 8 ? 4 : 2; }
+inline int64_t keyout_partial_bytes(int kw, int64_t n, int64_t C, int64_t Tk, int D) {
+  return n * keyout_tiles(kw, C, Tk) * (static_cast<int64_t>(D) * kTileQ * keyout_part_size(kw) + kTileQ * 4);
+}
+// Waves (32 keys each) per key group for a call: 16 or 8, whichever the measured
+// times put first.  A workgroup steps through its row tiles in 2.05 us each (16
+// waves) or 1.33 us (8 waves; two workgroups on a CU take 2.1 us per pair of
+// steps); the pass ends with its longest walk or, on a full chip, with its
+// steps over 256 CUs; the reduction reads the partials at 4.5 TB/s.  Measured, us
+// (pass + reduction, 16 / 8 waves): B2 H8 T4096 268 / 216, B3 H5 T1357 96 / 78,
+// B2 H4 T2048 135 / 101, B8 H16 T2048 212 / 252, B32 H12 T1024 215 / 240,
+// B1 H16 T16384 1336 / 1697.
+inline int keyout_waves(int64_t n, int64_t C, int64_t Tk, int D) {
+  auto us = [&](int kw, double step, double full_step) {
+    const double walk = static_cast<double>((C + kTileQ - 1) / kTileQ) * step;
+    const double full = static_cast<double>(n * keyout_tiles(kw, C, Tk)) / 256 * full_step;
+    return (walk > full ? walk : full) + static_cast<double>(keyout_partial_bytes(kw, n, C, Tk, D)) / 4.5e6;
+  };
+  // the small groups' partials are four times the room: at most 1 GiB of it
+  if (keyout_partial_bytes(8, n, C, Tk, D) > (int64_t{1} << 30)) return kKeyoutWaves;
+  return us(8, 1.33, 1.05) < us(16, 2.05, 2.05) ? 8 : 16;
 }
 inline bool keyout_eligible(int64_t C, int64_t Tk, int64_t q0, int D, int prec, bool requested) {
   return requested && prec == 2 && D == 64 && q0 + C == Tk && q0 % KeyGroups<kKeyoutWaves>::kKeys == 0 &&
-         keyout_partial_bytes(1, C, Tk, D) <= kKeyoutBudgetBytes;
+         keyout_partial_bytes(kKeyoutWaves, 1, C, Tk, D) <= kKeyoutBudgetBytes;
 }
 // slices per key-pass batch: all of them when their partials fit the budget,
 // else as many batches as the budget needs, of equal size (a last batch of a
 // slice or two would leave most CUs idle behind its longest walks)
-inline int64_t keyout_batch(int64_t n, int64_t C, int64_t Tk, int D) {
-  const int64_t per = keyout_partial_bytes(1, C, Tk, D);
+inline int64_t keyout_batch(int kw, int64_t n, int64_t C, int64_t Tk, int D) {
+  const int64_t per = keyout_partial_bytes(kw, 1, C, Tk, D);
   int64_t fit = per > 0 ? kKeyoutBudgetBytes / per : n;
   fit = fit < 1 ? 1 : (fit < n ? fit : n);
   const int64_t batches = (n + fit - 1) / fit;
@@ -1075,9 +1139,10 @@ FwdWorkspace fwd_layout(int64_t n, int64_t C, int64_t Tk, int D, int dtype, int 
   // the key pass's partials, when a chunk of this shape can take it (every
   // call is a chunk of rows [Tk - C, Tk) against keys [0, Tk))
   if (keyout_eligible(C, Tk, Tk - C, D, prec, key_pass)) {
-    const int64_t nb = keyout_batch(n, C, Tk, D);
-    w.rp = w.op + align_up(static_cast<size_t>(nb * keyout_tiles(C, Tk) * D * kTileQ * 2));
-    w.total = w.rp + align_up(static_cast<size_t>(nb * keyout_tiles(C, Tk) * kTileQ * 4));
+    const int kw = keyout_waves(n, C, Tk, D);
+    const int64_t tiles = keyout_batch(kw, n, C, Tk, D) * keyout_tiles(kw, C, Tk);
+    w.rp = w.op + align_up(static_cast<size_t>(tiles * D * kTileQ * keyout_part_size(kw)));
+    w.total = w.rp + align_up(static_cast<size_t>(tiles * kTileQ * 4));
   }
   return w;
 }
@@ -1166,12 +1231,13 @@ int launch_forward(const ForwardArgs& a) {
     if (key_pass) {
       // one key pass forms the checkpoints, the totals and the share V
       // partials; the reduction finishes out and ssum
-      __bf16* op = reinterpret_cast<__bf16*>(ws + w.op);
-      float* rp = reinterpret_cast<float*>(ws + w.rp);
-      constexpr int KW = kKeyoutWaves;
+      auto run = [&](auto kw) -> int {
+      constexpr int KW = decltype(kw)::value;
       using KG = KeyGroups<KW>;
+      KoPart<KW>* op = reinterpret_cast<KoPart<KW>*>(ws + w.op);
+      float* rp = reinterpret_cast<float*>(ws + w.rp);
       const unsigned nq = static_cast<unsigned>((a.C + kTileQ - 1) / kTileQ);
-      const int64_t ntiles = keyout_tiles(a.C, a.Tk);
+      const int64_t ntiles = keyout_tiles(KW, a.C, a.Tk);
       P.kgroups = static_cast<int>(KG::groups(a.Tk));
       // longest walks first, group by group, whatever the size: every chunk's
       // walks differ in length (its diagonal groups are shorter), and in slice
@@ -1181,7 +1247,7 @@ int launch_forward(const ForwardArgs& a) {
       // slices in batches whose partials fit the workspace (one batch at
       // every benchmark shape); each batch's pass and reduction see only its
       // slices, through pointers advanced to its first slice
-      const int64_t batch = keyout_batch(a.n, a.C, a.Tk, D);
+      const int64_t batch = keyout_batch(KW, a.n, a.C, a.Tk, D);
       for (int64_t b0 = 0; b0 < a.n; b0 += batch) {
         const int64_t nbat = min(batch, a.n - b0);
         FwdParams B = P;
@@ -1203,6 +1269,9 @@ int launch_forward(const ForwardArgs& a) {
         });
       }
       return static_cast<int>(hipGetLastError());
+      };
+      if (keyout_waves(a.n, a.C, a.Tk, D) == 8) return run(std::integral_constant<int, 8>{});
+      return run(std::integral_constant<int, 16>{});
     }
   }
   P.kgroups = static_cast<int>((a.Tk + 4 * kTileK - 1) / (4 * kTileK));

@@ -312,6 +312,9 @@ __device__ __forceinline__ bf16x8 load_once(const __bf16* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p));
 }
 __device__ __forceinline__ float load_once(const float* p) { return __builtin_nontemporal_load(p); }
+__device__ __forceinline__ floatx8 load8_once(const float* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const floatx8*>(p));
+}
 
 // The main loop of a double-buffered kernel: iter(i, buf) for i in [begin,
 // end), with LDS buffer buf = (i - begin) & 1.  UNROLL unrolls it by two so

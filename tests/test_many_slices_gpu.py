@@ -41,3 +41,26 @@ def test_decode_past_grid_y_limit():
     y = kernels.dilution_decode_step(q[:, :, t - 1:].contiguous().cuda(), k.cuda(), v.cuda(), committed, t)
     assert max_abs(y[:, :, 0], orc.attention_f64(q, k, v)[:, :, t - 1]) < 1e-4
     assert max_abs(committed, orc.demand_totals(q, k)) < 1e-5
+
+
+@pytest.mark.parametrize("seq", [1, 33, 255, 256, 257, 512, 545, 1024, 2049, 4097])
+def test_key_group_size_does_not_change_the_bits(seq):
+    """The forward's key pass takes groups of 256 or 512 keys by the size of the
+    call (keyout_waves); a slice's outputs, row sums and demand totals have the
+    same bits alone (256-key groups) and among many slices (512)."""
+    from dilution import kernels
+
+    many = max(64, 2 ** 18 // seq) if seq > 512 else 128
+    g = torch.Generator(device="cuda").manual_seed(seq)
+    q, k, v = (torch.randn(1, many, seq, 64, device="cuda", generator=g, dtype=torch.float32).to(torch.bfloat16)
+               for _ in range(3))
+    out, aux = kernels.dilution_attention_forward(q, k, v, dot_precision="bf16", return_aux=True)
+    for s in (0, many // 2, many - 1):
+        one, one_aux = kernels.dilution_attention_forward(q[:, s:s + 1], k[:, s:s + 1], v[:, s:s + 1],
+                                                          dot_precision="bf16", return_aux=True)
+        assert torch.equal(one[0, 0], out[0, s])
+        assert torch.equal(one_aux["ssum"][0], aux["ssum"][s])
+        assert torch.equal(one_aux["committed_total"][0, 0], aux["committed_total"][0, s])
+    # and those bits are right: the three-pass forward's, to bf16 partials
+    want = kernels.dilution_attention_reference(q[:, :1], k[:, :1], v[:, :1])
+    assert (out[:, :1] - want).abs().max() < 2e-2
