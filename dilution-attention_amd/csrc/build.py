@@ -4,7 +4,9 @@
 
 Each translation unit is compiled with hipcc into _build/ (git-ignored), then
 linked into dilution/libdilution_hip.so next to the Python package, in-tree, so
-the built library travels with the source tree.
+the built library travels with the source tree.  Beside it, dil_host.cpp (host code
+only) becomes the Python module dilution/_host.so against this interpreter's
+torch.
 """
 
 from __future__ import annotations
@@ -15,10 +17,12 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.join(os.path.dirname(HERE), "dilution")
 OUT = os.path.join(PKG, "libdilution_hip.so")
+HOST_OUT = os.path.join(PKG, "_host.so")
 BUILD = os.path.join(HERE, "_build")
 SOURCES = ["dil_api.hip", "dil_decode.hip", "dil_forward.hip", "dil_backward.hip", "dil_timing.hip",
            "dil_noalloc.hip", "dil_linear.hip"]
@@ -56,12 +60,33 @@ def _compile(unit) -> str:
     return obj
 
 
+def _build_host() -> str:
+    """dilution/_host.so, the native host side of the Python layer."""
+    import torch
+
+    root = os.path.dirname(os.path.abspath(torch.__file__))
+    include, lib = os.path.join(root, "include"), os.path.join(root, "lib")
+    tmp = HOST_OUT + ".tmp"
+    cmd = [os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-DTORCH_EXTENSION_NAME=_host",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-isystem", include,
+           "-isystem", os.path.join(include, "torch", "csrc", "api", "include"),
+           "-isystem", sysconfig.get_paths()["include"], os.path.join(HERE, "dil_host.cpp"), "-o", tmp,
+           f"-L{lib}", "-lc10", "-ltorch_cpu", "-ltorch_python"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for dil_host.cpp:\n{proc.stderr}")
+    os.replace(tmp, HOST_OUT)
+    return HOST_OUT
+
+
 def build(jobs: int | None = None, verbose: bool = False) -> str:
     os.makedirs(BUILD, exist_ok=True)
     units = [(os.path.splitext(src)[0], src, []) for src in SOURCES] + VARIANT_OBJECTS
     jobs = jobs or min(len(units), os.cpu_count() or 1)
     with cf.ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(_build_host)
         objs = list(pool.map(_compile, units))
+        host.result()
     tmp = OUT + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp]
     proc = subprocess.run(cmd, capture_output=True, text=True)
@@ -69,6 +94,7 @@ def build(jobs: int | None = None, verbose: bool = False) -> str:
         raise RuntimeError(f"link failed:\n{proc.stderr}")
     os.replace(tmp, OUT)
     if verbose:
+        print(f"built {HOST_OUT}")
         print(f"built {OUT}")
     return OUT
 

@@ -125,6 +125,12 @@ def lib():
     return handle
 
 
+def addresses() -> dict:
+    """{name: address} of the loaded library's entry points (for ``_host.bind``)."""
+    handle = lib()
+    return {name: ctypes.cast(getattr(handle, name), _vp).value for name in SIGNATURES}
+
+
 def check(status: int, what: str) -> None:
     if status != 0:
         msg = lib().dil_status_string(status).decode()

@@ -24,15 +24,22 @@ and ignored: tiles are fixed for gfx950.
 
 from __future__ import annotations
 
-import contextlib
 import math
 
 import torch
 
 from . import _hip
 
-HAS_HIP = _hip.available()
-"""True when libdilution_hip.so is built and loadable (the test gate)."""
+try:
+    from . import _host
+except ImportError as exc:              # not built, or built for another torch
+    _host, _host_error = None, str(exc)
+if _host is not None and _hip.available():
+    _host.bind(_hip.addresses())
+
+HAS_HIP = _hip.available() and _host is not None
+"""True when libdilution_hip.so and the native host module are built and
+loadable (the test gate)."""
 
 # The reference switches training above this length to its key-parallel
 # forward (kernels.py:71-76).  Here one decomposition serves every length; the
@@ -142,81 +149,20 @@ def _check_head_dim(head_dim: int, dot_precision: str | None = None) -> None:
                          f"(head_dim_supported(); got {dot_precision!r})")
 
 
-def _common_dtype(*ts: torch.Tensor) -> torch.dtype:
-    dt = ts[0].dtype
-    for t in ts[1:]:
-        dt = torch.promote_types(dt, t.dtype)
-    if dt not in _DTYPES:
-        dt = torch.float32
-    return dt
+def _native():
+    """The native host module: one call per entry point checks the arguments,
+    allocates and launches (csrc/dil_host.cpp)."""
+    if _host is None:
+        raise RuntimeError("dilution HIP kernels are not available: dilution/_host.so cannot be loaded "
+                           f"({_host_error}); run `python dilution-attention_amd/csrc/build.py`")
+    return _host
 
 
-def _rows(x: torch.Tensor, n: int, t: int, d: int, dtype: torch.dtype) -> torch.Tensor:
-    """(n, t, d) contiguous view or copy in `dtype` (kernels.py:362-364)."""
-    return x.reshape(n, t, d).to(dtype).contiguous()
-
-
-def _strided_rows(x: torch.Tensor) -> bool:
-    """Whether the kernels read (or write) this (B, H, T, D) tensor where it
-    lies (the layout rules of ``dil_rows``): contiguous head dims, rows and
-    slices at 16-byte steps, the row stride from head_dim to 2^20 elements.
-    Rows that are apart also have to lie within 2^31 bytes, which the one-pass
-    backward's 32-bit offsets cover."""
-    batch, heads, seq, head_dim = x.shape
-    sb, sh, st, sd = x.stride()
-    es = x.element_size()
-    lane = 16 // es
-    return (sd == 1 and head_dim <= st < (1 << 20) and st % lane == 0
-            and (batch == 1 or sb % lane == 0) and (heads == 1 or sh % lane == 0)
-            and (st == head_dim or seq * st * es < (1 << 31)) and x.data_ptr() % 16 == 0)
-
-
-def _operand(x: torch.Tensor, dtype: torch.dtype, flat: bool = False) -> torch.Tensor:
-    """x (B, H, T, D) in `dtype` as the kernels can read it: x itself when
-    its type and layout allow (views of a fused projection do), else a
-    contiguous copy.  `flat`: rows head_dim apart."""
-    x = x.to(dtype)
-    if flat:
-        x = x.contiguous()
-    return x if _strided_rows(x) else x.clone(memory_format=torch.contiguous_format)
-
-
-def _slice_dims(batch: int, heads: int) -> tuple[int, int]:
-    """(batch, heads) as the kernels count slices: as they are within
-    ``dil_rows``' limits, else every slice a batch of its own."""
-    if heads < 1 << 16 and batch * heads * heads < 1 << 32:
-        return batch, heads
-    return batch * heads, 1
-
-
-def _sliced(x: torch.Tensor, dims: tuple[int, int]) -> torch.Tensor:
-    """x (B, H, T, D) with its slices counted as `dims`."""
-    if x.shape[:2] == dims:
-        return x
-    return x.contiguous().view(*dims, *x.shape[2:])
-
-
-def _flat_only(variant: tuple, head_dim: int) -> bool:
-    """The calls whose kernels are built for rows head_dim apart only: the
-    ablation variants, and head_dim 256 (no registers for a row stride)."""
-    return head_dim > 128 or tuple(variant) != _PRODUCTION
-
-
-def _row_ref(x: torch.Tensor):
-    """``dil_rows`` of a (B, H, T, D) tensor that ``_strided_rows`` accepts."""
-    sb, sh, st, _ = x.stride()
-    return _hip.Rows(x.data_ptr(), sb, sh, st)
-
-
-def _empty_as(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
-    """A new (B, H, T, D) tensor in `dtype` whose memory order follows x:
-    (B, T, H, D) when x's rows are stepped over heads first (the views of a
-    (B, T, H * D) projection), so that its view back to (B, T, H * D) needs no
-    copy; else contiguous."""
-    batch, heads, seq, head_dim = x.shape
-    if heads > 1 and seq > 1 and x.stride(1) < x.stride(2):
-        return torch.empty(batch, seq, heads, head_dim, device=x.device, dtype=dtype).transpose(1, 2)
-    return torch.empty(batch, heads, seq, head_dim, device=x.device, dtype=dtype)
+def _raw_stream(x: torch.Tensor) -> int:
+    """The current stream of x's device, as its raw handle (0 for a CPU
+    tensor, which the native checks refuse)."""
+    idx = x.get_device()
+    return torch._C._cuda_getCurrentRawStream(idx) if idx >= 0 else 0
 
 
 def _stream(dev: torch.device) -> int:
@@ -225,20 +171,6 @@ def _stream(dev: torch.device) -> int:
     asks for it about 60 times.)"""
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
     return torch._C._cuda_getCurrentRawStream(idx)
-
-
-_NO_SWITCH = contextlib.nullcontext()
-
-
-def _on(dev: torch.device):
-    """The inputs' device made current for a launch; no switch when it already is."""
-    if dev.index is None or dev.index == torch.cuda.current_device():
-        return _NO_SWITCH
-    return torch.cuda.device(dev)
-
-
-def _ptr(t: torch.Tensor | None) -> int | None:
-    return None if t is None else t.data_ptr()
 
 
 def _workspace(nbytes: int, device) -> torch.Tensor:
@@ -279,60 +211,14 @@ def dilution_attention_forward(
     checkpoint scratch stays under scratch_budget_gib; slices are independent,
     so results are identical either way.
     """
-    prec = _precision_code(dot_precision)
-    if q.dim() != 4 or q.shape != k.shape or q.shape != v.shape:
-        raise ValueError(f"q, k, v must share one (B, H, T, D) shape, got {tuple(q.shape)}, "
-                         f"{tuple(k.shape)}, {tuple(v.shape)}")
-    batch, heads, seq, head_dim = q.shape
-    _check_head_dim(head_dim, dot_precision)
-    _check_device(q, k, v)
-    lib = _hip.lib()
-    n = batch * heads
-    dt = _common_dtype(q, k, v)
-    qf, kf, vf = (_operand(x, dt, _flat_only(_variant, head_dim)) for x in (q, k, v))
-    dev = q.device
-    nb = (seq + CHECKPOINT_ROWS - 1) // CHECKPOINT_ROWS
-    f32 = dict(device=dev, dtype=torch.float32)
-    out = torch.empty(n, seq, head_dim, **f32)
-    rmax = torch.empty(n, seq, **f32)
-    rden = torch.empty(n, seq, **f32)
-    ssum = torch.empty(n, seq, **f32)
-    total = torch.empty(n, seq, **f32)
-    pk = torch.empty(n, seq, head_dim, **f32) if _save_pk else None
-
-    rows = n
-    carry = None
+    _precision_code(dot_precision)
+    out, rmax, rden, ssum, total, pk, carry = _native().forward(
+        q, k, v, dot_precision, return_aux, _save_pk, scratch_budget_gib, _variant, _raw_stream(q))
     if return_aux:
-        carry = torch.empty(n, nb, seq, **f32)
-    elif tuple(_variant) != _PRODUCTION or not lib.dil_forward_key_pass(seq, 0, head_dim, _DTYPES[dt], prec):
-        # the three-pass forward reads the checkpoints it writes: the slices go
-        # in groups whose (rows, T/32, T) scratch fits the budget.  The key pass
-        # writes none without aux and takes every slice in one call.
-        per_row = nb * seq * 4
-        rows = max(1, min(n, int(scratch_budget_gib * 2**30) // max(per_row, 1)))
-        carry = torch.empty(rows, nb, seq, **f32)
-    ws_bytes = lib.dil_forward_workspace_bytes(rows, seq, head_dim, _DTYPES[dt], prec, int(_save_pk))
-    ws = _workspace(ws_bytes, dev)
-    dims = _slice_dims(batch, heads) if rows >= n else (n, 1)   # (n, 1): groups of slices
-    qf, kf, vf = (_sliced(x, dims) for x in (qf, kf, vf))
-    for a in range(0, n, rows):
-        b = min(a + rows, n)
-        part = (qf, kf, vf) if rows >= n else tuple(x[a:b] for x in (qf, kf, vf))
-        with _on(dev):
-            status = lib.dil_forward_rows(
-                *(_row_ref(x) for x in part), *part[0].shape[:2], seq, head_dim, _DTYPES[dt], prec, *_variant,
-                out[a:b].data_ptr(), rmax[a:b].data_ptr(), rden[a:b].data_ptr(), ssum[a:b].data_ptr(),
-                _ptr(carry), total[a:b].data_ptr(), None if pk is None else pk[a:b].data_ptr(),
-                ws.data_ptr(), ws.numel(), _stream(dev))
-        _hip.check(status, "dil_forward")
-
-    result = out.reshape(batch, heads, seq, head_dim)
-    if return_aux:
-        aux = dict(pk=pk, rmax=rmax, rden=rden, carry=carry, ssum=ssum, bwd_block_m=CHECKPOINT_ROWS,
-                   block_m=block_m, block_n=block_n, dot_precision=dot_precision,
-                   num_warps=num_warps, committed_total=total.reshape(batch, heads, seq))
-        return result, aux
-    return result
+        return out, dict(pk=pk, rmax=rmax, rden=rden, carry=carry, ssum=ssum, bwd_block_m=CHECKPOINT_ROWS,
+                         block_m=block_m, block_n=block_n, dot_precision=dot_precision, num_warps=num_warps,
+                         committed_total=total)
+    return out
 
 
 # ---------------------------------------------------------------------------
@@ -370,30 +256,7 @@ class _DilutionAttentionFn(torch.autograd.Function):
 
 def _backward(saved, dout, dot_precision: str, variant: tuple):
     """dq, dk, dv of the operator (variant) from the forward's saved tensors."""
-    q, k, v, out, rmax, rden, carry, ssum, pk = saved
-    lib = _hip.lib()
-    batch, heads, seq, head_dim = q.shape
-    n = batch * heads
-    prec = _precision_code(dot_precision)
-    dt = _common_dtype(q, k, v)
-    qf, kf, vf = (_operand(x, dt, _flat_only(variant, head_dim)) for x in (q, k, v))
-    ddt = dout.dtype if dout.dtype in _DTYPES else torch.float32
-    dof = _operand(dout.reshape(q.shape), ddt)
-    dev = q.device
-    dims = _slice_dims(batch, heads)
-    qf, kf, vf, dof = (_sliced(x, dims) for x in (qf, kf, vf, dof))
-    # the gradients in the memory order of their inputs
-    dq, dk, dv = (_sliced(_empty_as(x, dt), dims) for x in (q, k, v))
-    ws = _workspace(lib.dil_backward_workspace_bytes(n, seq, head_dim, _DTYPES[dt], prec), dev)
-    with _on(dev):
-        status = lib.dil_backward_rows(
-            _row_ref(qf), _row_ref(kf), _row_ref(vf), _row_ref(dof), out.data_ptr(), rmax.data_ptr(),
-            rden.data_ptr(), ssum.data_ptr(), carry.data_ptr(), pk.data_ptr(), *dims, seq, head_dim,
-            _DTYPES[dt], _DTYPES[ddt], _DTYPES[dt], prec, *variant, _row_ref(dq), _row_ref(dk), _row_ref(dv),
-            ws.data_ptr(), ws.numel(), _stream(dev))
-    _hip.check(status, "dil_backward")
-    return tuple(g.view(ref.shape).to(ref.dtype) if dims != ref.shape[:2] else g.to(ref.dtype)
-                 for g, ref in zip((dq, dk, dv), (q, k, v)))
+    return _native().backward(*saved, dout, dot_precision, variant, _raw_stream(dout))
 
 
 def dilution_attention(
@@ -451,46 +314,12 @@ def dilution_prefill_chunk(
     ``_strided_rows`` accepts, any float dtype) takes the outputs in place of a
     new fp32 tensor.
     """
-    prec = _precision_code(dot_precision)
-    capacity = _check_cache(q, k_cache, v_cache, committed)
-    batch, heads, chunk, head_dim = q.shape
-    _check_head_dim(head_dim, dot_precision)
-    if start < 0 or start + chunk > capacity:
-        raise ValueError(f"rows [{start}, {start + chunk}) outside cache capacity {capacity}")
-    _check_device(q, k_cache, v_cache, committed)
-    lib = _hip.lib()
-    n = batch * heads
-    dt = k_cache.dtype if k_cache.dtype in _DTYPES else torch.float32
-    if v_cache.dtype != dt or k_cache.dtype != dt:
-        raise ValueError("k_cache and v_cache must share a float dtype")
-    kf = k_cache.view(n, capacity, head_dim)
-    vf = v_cache.view(n, capacity, head_dim)
-    cf = committed.view(n, capacity)
-    qf = _operand(q, dt, _flat_only(_PRODUCTION, head_dim))
-    dev = q.device
-    nb = (chunk + CHECKPOINT_ROWS - 1) // CHECKPOINT_ROWS
-    f32 = dict(device=dev, dtype=torch.float32)
-    out = torch.empty(batch, heads, chunk, head_dim, **f32) if _out is None else _out
-    rmax = torch.empty(n, chunk, **f32)
-    rden = torch.empty(n, chunk, **f32)
-    ssum = torch.empty(n, chunk, **f32)
-    # the key pass writes the checkpoints only for a caller that keeps them
-    carry = None
-    if return_aux or not lib.dil_forward_key_pass(chunk, start, head_dim, _DTYPES[dt], prec):
-        carry = torch.empty(n, nb, start + chunk, **f32)
-    ws = _workspace(lib.dil_prefill_workspace_bytes(n, chunk, start, head_dim, _DTYPES[dt], prec), dev)
-    dims = _slice_dims(batch, heads)
-    qf = _sliced(qf, dims)
-    rows = out if dims == out.shape[:2] else out.view(*dims, chunk, head_dim)
-    with _on(dev):
-        status = lib.dil_prefill_rows(
-            _row_ref(qf), kf.data_ptr(), vf.data_ptr(), *dims, chunk, start, capacity, head_dim,
-            _DTYPES[dt], prec, cf.data_ptr(), _row_ref(rows), _DTYPES[out.dtype], rmax.data_ptr(),
-            rden.data_ptr(), ssum.data_ptr(), _ptr(carry), ws.data_ptr(), ws.numel(), _stream(dev))
-    _hip.check(status, "dil_prefill_chunk")
+    _precision_code(dot_precision)
+    out, rmax, rden, ssum, carry = _native().prefill_chunk(
+        q, k_cache, v_cache, committed, start, dot_precision, return_aux, _out, _raw_stream(q))
     if return_aux:
         return out, dict(rmax=rmax, rden=rden, ssum=ssum, carry=carry,
-                            bwd_block_m=CHECKPOINT_ROWS, dot_precision=dot_precision)
+                         bwd_block_m=CHECKPOINT_ROWS, dot_precision=dot_precision)
     return out
 
 
@@ -518,42 +347,7 @@ def dilution_decode_step(
     must be zero).  It is advanced in place to include this row; positions
     >= length are never touched.
     """
-    batch, heads, one, head_dim = q1.shape
-    if one != 1:
-        raise ValueError("decode step takes exactly one query row per (batch, head)")
-    if head_dim & (head_dim - 1):
-        raise ValueError("head_dim must be a power of two")
-    capacity = _check_cache(q1, k_cache, v_cache, committed)
-    if not 1 <= length <= capacity:
-        raise ValueError(f"length {length} outside cache capacity {capacity}")
-    _check_head_dim(head_dim)
-    _check_device(q1, k_cache, v_cache, committed)
-    lib = _hip.lib()
-    n = batch * heads
-    dt = k_cache.dtype if k_cache.dtype in _DTYPES else torch.float32
-    if v_cache.dtype != dt or k_cache.dtype != dt:
-        raise ValueError("k_cache and v_cache must share a float dtype")
-    kf = k_cache.view(n, capacity, head_dim)
-    vf = v_cache.view(n, capacity, head_dim)
-    cf = committed.view(n, capacity)
-    # q1 keeps its own dtype: the kernels read it as fp32 and store the
-    # output in it (kernels.py:953, 1029)
-    qdt = q1.dtype if q1.dtype in _DTYPES else torch.float32
-    qf = q1.reshape(n, head_dim).to(qdt).contiguous()
-    out = torch.empty(n, head_dim, device=q1.device, dtype=qdt)
-    ws = _workspace(lib.dil_decode_workspace_bytes(n, length, head_dim), q1.device)
-    head = (qf.data_ptr(), kf.data_ptr(), vf.data_ptr(), cf.data_ptr(), out.data_ptr(), n,
-            capacity, length, head_dim, _DTYPES[dt], _DTYPES[qdt])
-    tail = (ws.data_ptr(), ws.numel(), _stream(q1.device))
-    with _on(q1.device):
-        if tuple(_variant) == _PRODUCTION:
-            status = lib.dil_decode_step(*head, *tail)
-        else:
-            status = lib.dil_decode_step_variant(*head, *_variant, *tail)
-    _hip.check(status, "dil_decode_step")
-    if out.dtype != q1.dtype:
-        out = out.to(q1.dtype)
-    return out.view(batch, heads, 1, head_dim)
+    return _native().decode_step(q1, k_cache, v_cache, committed, length, _variant, _raw_stream(q1))
 
 
 def decode_step_device_length(q1: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,

@@ -62,39 +62,7 @@ def rows_linear(x: torch.Tensor, w1: torch.Tensor, mode: int, *, w2: torch.Tenso
     silu(r W1^T) * (r W2^T) with r = rmsnorm(x; g, eps), rounded to bf16 where
     the separate torch ops round.  (No reference counterpart: the reference
     model runs these through torch.nn.Linear, model.py:41-93.)"""
-    if x.dim() != 2 or w1.dim() != 2:
-        raise ValueError("rows_linear takes x (rows, K) and a weight (N, K)")
-    rows, k = x.shape
-    n = w1.shape[0]
-    for t in (x, w1, w2, g, resid):
-        if t is not None and (t.dtype != torch.bfloat16 or not t.is_contiguous() or t.device != x.device):
-            raise ValueError("rows_linear takes contiguous bf16 tensors on one device")
-    # the kernel indexes every operand with the rows, N and K given here
-    if w1.shape[1] != k:
-        raise ValueError(f"rows_linear: weight {tuple(w1.shape)} does not match x {tuple(x.shape)}")
-    if w2 is not None and w2.shape != w1.shape:
-        raise ValueError(f"rows_linear: w2 {tuple(w2.shape)} must have w1's shape {tuple(w1.shape)}")
-    if g is not None and g.shape != (k,):
-        raise ValueError(f"rows_linear: the norm weight must have shape ({k},), got {tuple(g.shape)}")
-    if resid is not None and resid.shape != (rows, n):
-        raise ValueError(f"rows_linear: resid must have shape ({rows}, {n}), got {tuple(resid.shape)}")
-    if mode in (_LIN_NORM, _LIN_SWIGLU) and g is None:
-        raise ValueError("rows_linear: the normed modes need the norm weight g")
-    if mode == _LIN_SWIGLU and w2 is None:
-        raise ValueError("rows_linear: the SwiGLU mode needs w2")
-    if mode == _LIN_RESID and resid is None:
-        raise ValueError("rows_linear: the residual mode needs resid")
-    lib = _hip.lib()
-    if out is None:
-        out = torch.empty(rows, n, device=x.device, dtype=x.dtype)
-    elif out.shape != (rows, n) or out.dtype != torch.bfloat16 or not out.is_contiguous() or out.device != x.device:
-        raise ValueError("out must be a contiguous bf16 (rows, N) tensor on the inputs' device")
-    status = lib.dil_rows_linear(x.data_ptr(), w1.data_ptr(), None if w2 is None else w2.data_ptr(),
-                                 None if g is None else g.data_ptr(), None if resid is None else resid.data_ptr(),
-                                 out.data_ptr(), rows, n, k, mode, 1, float(eps),
-                                 kernels._stream(x.device))
-    _hip.check(status, "dil_rows_linear")
-    return out
+    return kernels._native().rows_linear(x, w1, mode, w2, g, resid, eps, out, kernels._raw_stream(x))
 
 
 def rows_linear_qkv(x: torch.Tensor, w: torch.Tensor, g: torch.Tensor, eps: float, k_cache: torch.Tensor,
@@ -107,30 +75,8 @@ def rows_linear_qkv(x: torch.Tensor, w: torch.Tensor, g: torch.Tensor, eps: floa
     the kernel runs, as in a graph replay).  (No reference counterpart: the
     reference projects with c_attn and writes its cache as separate ops,
     model.py:41-93.)"""
-    if x.dim() != 2 or k_cache.dim() != 4:
-        raise ValueError("rows_linear_qkv takes x (B, d_model) and (B, H, capacity, D) caches")
-    rows, k = x.shape
-    batch, heads, capacity, head_dim = k_cache.shape
-    for t in (x, w, g, k_cache, v_cache):
-        if t.dtype != torch.bfloat16 or not t.is_contiguous() or t.device != x.device:
-            raise ValueError("rows_linear_qkv takes contiguous bf16 tensors on one device")
-    if batch != rows or v_cache.shape != k_cache.shape or w.shape != (3 * heads * head_dim, k):
-        raise ValueError("rows_linear_qkv: x, w and the caches disagree in shape")
-    if g.shape != (k,):
-        raise ValueError(f"rows_linear_qkv: the norm weight must have shape ({k},), got {tuple(g.shape)}")
-    lib = _hip.lib()
-    q = torch.empty(rows, heads * head_dim, device=x.device, dtype=x.dtype)
-    if torch.is_tensor(pos):
-        if pos.dtype != torch.int64 or pos.numel() != 1 or pos.device != x.device:
-            raise ValueError("a device position is a one-element int64 tensor on the inputs' device")
-        pos_dev, pos_host = pos.data_ptr(), 0
-    else:
-        pos_dev, pos_host = None, int(pos)
-    status = lib.dil_rows_linear_qkv(x.data_ptr(), w.data_ptr(), g.data_ptr(), q.data_ptr(), k_cache.data_ptr(),
-                                     v_cache.data_ptr(), rows, heads, head_dim, capacity, pos_dev, pos_host, k, 1,
-                                     float(eps), kernels._stream(x.device))
-    _hip.check(status, "dil_rows_linear_qkv")
-    return q
+    dev, host = (pos, 0) if torch.is_tensor(pos) else (None, int(pos))
+    return kernels._native().rows_linear_qkv(x, w, g, eps, k_cache, v_cache, dev, host, kernels._raw_stream(x))
 
 
 def rows_argmax(logits: torch.Tensor, limit: int | None = None, out: torch.Tensor | None = None) -> torch.Tensor:

@@ -32,6 +32,10 @@ def _packed(x, width, at):
     return view
 
 
+def _rows(x):
+    return _hip.Rows(x.data_ptr(), *x.stride()[:3])
+
+
 def _inputs(shape, dtype, device="cuda"):
     g = torch.Generator().manual_seed(5)
     xs = [torch.randn(shape, generator=g) * s for s in (0.5, 0.5, 1.0)]
@@ -47,26 +51,26 @@ def test_rule_matches_the_library(layout):
     x = LAYOUTS[layout](torch.randn(2, 3, 40, 64).to(torch.bfloat16))
     lib = _hip.lib()
     fake = [ctypes.c_void_p(0x1000 * (i + 1)) for i in range(8)]
-    row = kernels._row_ref(x)
+    row = _rows(x)
     status = lib.dil_forward_rows(row, row, row, 2, 3, 40, 64, 1, 2, 0, 1, 1.0, *fake[:6], None, fake[6], 0, None)
-    taken = kernels._strided_rows(x) and x.stride(3) == 1
+    taken = kernels._native().strided_rows(x) and x.stride(3) == 1
     assert taken == (layout not in ("misaligned", "dthb", "row_major_t"))
     if x.stride(3) == 1:                      # the library is told nothing of the head dims' stride
         assert status == (-3 if taken else -4)
 
 
 def test_slice_limits_and_gradient_order():
-    assert kernels._slice_dims(4, 16) == (4, 16)
-    assert kernels._slice_dims(3, 1 << 16) == (3 << 16, 1)
-    assert kernels._slice_dims(200, 10000) == (200 * 10000, 1)
+    assert kernels._native().slice_dims(4, 16) == (4, 16)
+    assert kernels._native().slice_dims(3, 1 << 16) == (3 << 16, 1)
+    assert kernels._native().slice_dims(200, 10000) == (200 * 10000, 1)
     lib = _hip.lib()
     x = torch.zeros(1, 1, 8, 64, dtype=torch.bfloat16)
-    row = kernels._row_ref(x)
+    row = _rows(x)
     assert lib.dil_forward_rows(row, row, row, 200, 10000, 8, 64, 1, 2, 0, 1, 1.0, *[None] * 8, 0, None) == -4
     packed = LAYOUTS["packed"](torch.zeros(2, 3, 5, 64))
-    grad = kernels._empty_as(packed, torch.float32)
+    grad = kernels._native().empty_as(packed, torch.float32)
     assert grad.shape == packed.shape and grad.transpose(1, 2).is_contiguous()
-    assert kernels._empty_as(LAYOUTS["hbtd"](torch.zeros(2, 3, 5, 64)), torch.float32).is_contiguous()
+    assert kernels._native().empty_as(LAYOUTS["hbtd"](torch.zeros(2, 3, 5, 64)), torch.float32).is_contiguous()
 
 
 def _train(q, k, v, dout, prec, ops=kernels, **kw):
