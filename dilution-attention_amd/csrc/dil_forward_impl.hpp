@@ -1108,6 +1108,20 @@ inline bool keyout_eligible(int64_t C, int64_t Tk, int64_t q0, int D, int prec, 
   return requested && prec == 2 && D == 64 && q0 + C == Tk && q0 % KeyGroups<kKeyoutWaves>::kKeys == 0 &&
          keyout_partial_bytes(kKeyoutWaves, 1, C, Tk, D) <= kKeyoutBudgetBytes;
 }
+// Whether a call that could take the key pass runs the three-pass forward
+// instead: short rows and few of them.  There the key pass's walks are a serial
+// chain on a few CUs (2.05 or 1.33 us per 32-row tile), where fwd_demand's walks
+// are one score product and one exp2 sweep per tile (~0.5 us) and fwd_out spreads
+// over the rows.  Measured, us (fwd_demand + fwd_out, key pass + reduction):
+// B1 H4 T512 30 / 35, B3 H5 T1357 60 / 78, B1 H16 T2048 83 / 105, B4 H16 T2048
+// 125 / 153, B4 H16 T1024 52 / 69, B16 H16 T256 26 / 31; beyond 2^17 tokens the
+// lead is gone (B8 H16 T2048 222 + 9 of V^T / 208).  Rows of more than 2048 keys
+// keep the key pass (its bits: a prefix has those of the whole sequence).
+// Without pk the three-pass forward's V^T is a launch of its own (~5 us), which
+// rows of up to 256 keys do not earn back.
+inline bool few_short_rows(int64_t n, int64_t Tk, bool pk) {
+  return Tk <= 2048 && n * Tk <= (int64_t{1} << 17) && (pk || Tk > 256);
+}
 // slices per key-pass batch: all of them when their partials fit the budget,
 // else as many batches as the budget needs, of equal size (a last batch of a
 // slice or two would leave most CUs idle behind its longest walks)
@@ -1120,7 +1134,7 @@ inline int64_t keyout_batch(int kw, int64_t n, int64_t C, int64_t Tk, int D) {
 }
 
 struct FwdWorkspace {
-  size_t vt, kt, qc, kc, op, rp, total;
+  size_t vt, kt, qc, kc, op, rp, carry, total;
 };
 
 FwdWorkspace fwd_layout(int64_t n, int64_t C, int64_t Tk, int D, int dtype, int prec, int want_pk,
@@ -1135,10 +1149,14 @@ FwdWorkspace fwd_layout(int64_t n, int64_t C, int64_t Tk, int D, int dtype, int 
   w.kc = w.qc + (convert ? align_up(ct * n * C * D) : 0);
   w.op = w.kc + (convert ? align_up(ct * n * Tk * D) : 0);
   w.rp = w.op;
+  w.carry = w.op;
   w.total = w.op;
   // the key pass's partials, when a chunk of this shape can take it (every
   // call is a chunk of rows [Tk - C, Tk) against keys [0, Tk))
-  if (keyout_eligible(C, Tk, Tk - C, D, prec, key_pass)) {
+  if (keyout_eligible(C, Tk, Tk - C, D, prec, key_pass) && few_short_rows(n, Tk, want_pk != 0)) {
+    // the three-pass forward's checkpoints, for a caller that keeps none
+    w.total = w.carry + align_up(static_cast<size_t>(4 * n * ((C + kTileQ - 1) / kTileQ) * Tk));
+  } else if (keyout_eligible(C, Tk, Tk - C, D, prec, key_pass)) {
     const int kw = keyout_waves(n, C, Tk, D);
     const int64_t tiles = keyout_batch(kw, n, C, Tk, D) * keyout_tiles(kw, C, Tk);
     w.rp = w.op + align_up(static_cast<size_t>(tiles * D * kTileQ * keyout_part_size(kw)));
@@ -1163,7 +1181,8 @@ int launch_forward(const ForwardArgs& a) {
   // workspace keeps its room, shared with the three-pass forward's layout)
   constexpr bool kKeyPassBuilt =
       std::is_same_v<CT, __bf16> && D == 64 && BID == BID_SOFTMAX && SHARE == SHARE_INCL;
-  const bool key_pass = kKeyPassBuilt && keyout_eligible(a.C, a.Tk, a.q0, D, kOperandPrec<CT>, a.key_pass);
+  const bool could = kKeyPassBuilt && keyout_eligible(a.C, a.Tk, a.q0, D, kOperandPrec<CT>, a.key_pass);
+  const bool key_pass = could && !few_short_rows(a.n, a.Tk, a.pk != nullptr);
   const bool v_rows = key_pass && !convert;
 
   // operands in the compute type; V^T (and K^T) tiles
@@ -1210,7 +1229,7 @@ int launch_forward(const ForwardArgs& a) {
   P.rmax = a.rmax;
   P.rden = a.rden;
   P.ssum = a.ssum;
-  P.carry = a.carry;
+  P.carry = a.carry == nullptr && could && !key_pass ? reinterpret_cast<float*>(ws + w.carry) : a.carry;
   P.demand_in = a.demand_in;
   P.din_sn = a.din_sn;
   P.total = a.total;

@@ -43,14 +43,15 @@ def test_decode_past_grid_y_limit():
     assert max_abs(committed, orc.demand_totals(q, k)) < 1e-5
 
 
-@pytest.mark.parametrize("seq", [1, 33, 255, 256, 257, 512, 545, 1024, 2049, 4097])
+@pytest.mark.parametrize("seq", [2049, 2560, 4097])
 def test_key_group_size_does_not_change_the_bits(seq):
-    """The forward's key pass takes groups of 256 or 512 keys by the size of the
-    call (keyout_waves); a slice's outputs, row sums and demand totals have the
-    same bits alone (256-key groups) and among many slices (512)."""
+    """Above 2048 keys the forward's key pass takes groups of 256 or 512 keys
+    by the size of the call (keyout_waves); a slice's outputs, row sums and
+    demand totals have the same bits alone (256-key groups) and among many
+    slices (512)."""
     from dilution import kernels
 
-    many = max(64, 2 ** 18 // seq) if seq > 512 else 128
+    many = 2 ** 19 // seq
     g = torch.Generator(device="cuda").manual_seed(seq)
     q, k, v = (torch.randn(1, many, seq, 64, device="cuda", generator=g, dtype=torch.float32).to(torch.bfloat16)
                for _ in range(3))
@@ -61,6 +62,30 @@ def test_key_group_size_does_not_change_the_bits(seq):
         assert torch.equal(one[0, 0], out[0, s])
         assert torch.equal(one_aux["ssum"][0], aux["ssum"][s])
         assert torch.equal(one_aux["committed_total"][0, 0], aux["committed_total"][0, s])
-    # and those bits are right: the three-pass forward's, to bf16 partials
-    want = kernels.dilution_attention_reference(q[:, :1], k[:, :1], v[:, :1])
-    assert (out[:, :1] - want).abs().max() < 2e-2
+
+
+@pytest.mark.parametrize("heads,seq,pk", [(1, 1, True), (3, 33, True), (4, 257, False), (4, 256, False), (64, 2048, True),
+                                          (65, 2048, True), (2, 2048, False), (512, 256, True), (513, 256, True)])
+def test_few_short_rows_forward(heads, seq, pk):
+    """Few short rows take the three-pass forward (few_short_rows), the others
+    the key pass: on both sides of each limit of the rule the outputs, the row
+    sums and the demand are the reference's, with and without checkpoints kept,
+    and a call without aux has the bits of the call with it."""
+    from dilution import kernels
+
+    g = torch.Generator(device="cuda").manual_seed(seq + heads)
+    q, k, v = (torch.randn(1, heads, seq, 64, device="cuda", generator=g, dtype=torch.float32).to(torch.bfloat16)
+               for _ in range(3))
+    out, aux = kernels.dilution_attention_forward(q, k, v, dot_precision="bf16", return_aux=True, _save_pk=pk)
+    if not pk:
+        assert torch.equal(out, kernels.dilution_attention_forward(q, k, v, dot_precision="bf16"))
+    for s in sorted({0, heads // 2, heads - 1}):
+        xs = [x[:, s:s + 1].double() for x in (q, k, v)]
+        a = (xs[0] @ xs[1].transpose(-1, -2).contiguous()) / 8
+        p = a.masked_fill(torch.ones(seq, seq, dtype=torch.bool, device="cuda").triu(1), float("-inf")).softmax(-1)
+        total = p.cumsum(-2)
+        share = p / (total + 1e-9)
+        want = (share / (share.sum(-1, keepdim=True) + 1e-9)) @ xs[2]
+        assert (out[:, s:s + 1] - want).abs().max() < 2e-2
+        assert ((aux["ssum"][s] - share.sum(-1)[0, 0]) / share.sum(-1)[0, 0]).abs().max() < 1e-2
+        assert (aux["committed_total"][:, s] - total[:, 0, -1]).abs().max() < 1e-5 * max(1, seq ** 0.5)
