@@ -42,6 +42,7 @@
 #include "dil_internal.hpp"
 #include "dil_tiles.hpp"
 #include "dil_variant.hpp"
+#include "dil_walk.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -236,7 +237,8 @@ constexpr int bwd_occupancy() {
 // the parked form is 8 waves (256 rows) per workgroup: <= 256 registers a
 // lane (two waves per SIMD, where the register form holds one) and ~124 KB
 // of LDS (the parked dO' of 8 waves and one set of K / V / K^T stages for
-// all of them), one workgroup per CU.
+// all of them), one workgroup per CU; 4 waves (~90 KB) where 8-wave groups
+// leave CUs idle (query_few).
 template <typename CT, int D>
 constexpr bool query_parks() {
   return D <= 64;
@@ -245,6 +247,16 @@ template <typename CT, int D>
 constexpr int query_waves() {
   return sizeof(CT) == 2 ? 4 : 8;
 }
+template <typename CT, int D, bool PARK>
+constexpr int query_occupancy() {                    // workgroups per CU asked of the compiler
+  return PARK && query_parks<CT, D>() ? (sizeof(CT) == 2 ? 3 : 1) : bwd_occupancy<CT, D>();
+}
+// Whether the 8-wave form runs as 4-wave workgroups: up to one 8-wave group per
+// CU (256 x 8 tiles) their number and their unequal walks bound the pass.  us,
+// 8 -> 4 waves: fp32 64 1024 tiles 465 -> 283, 2048 469 -> 314, 4096 536 -> 625;
+// fp32 32 2048 tiles 302 -> 236; split 64 1024 tiles 153 -> 121, 2048 157 -> 141,
+// 3072 161 -> 223; split 32 1536 tiles 117 -> 93.
+inline bool query_few(int64_t n, int64_t tiles) { return n * tiles <= 2048; }
 
 // ---------------------------------------------------------------------------
 // key-parallel reverse pass: dv, dk_main, suffix checkpoints
@@ -504,8 +516,7 @@ __global__ __launch_bounds__(kThreads, (bwd_occupancy<CT, D>())) void bwd_key(Bw
 
 template <typename CT, int D, int BID = BID_SOFTMAX, int SHARE = SHARE_INCL, bool PARK = false,
           int W = 4, bool FLAT = true>
-__global__ __launch_bounds__(64 * W, ((PARK && query_parks<CT, D>()) ? (W == 4 ? 3 : 1) : bwd_occupancy<CT, D>())) void bwd_query(
-    BwdParams P) {
+__global__ __launch_bounds__(64 * W, (query_occupancy<CT, D, PARK>())) void bwd_query(BwdParams P) {
   using TL = Tiles<CT, D>;
   using Frag = typename Mma<CT>::frag;
   constexpr int kNS = BID == BID_SOFTMAX ? 2 : 3;                // per-row statistics staged
@@ -959,6 +970,82 @@ __global__ __launch_bounds__(kThreads, (sizeof(CT) == 2 && D <= 64) ? 3 : 2) voi
           store4_as(P.dk, out + d, P.gdt, v);
         }
       }
+  }
+}
+
+// bwd_dkcorr with its walk split over the waves (dil_walk.hpp): one workgroup per
+// 32 keys, wave w takes every fourth row tile from the diagonal on, and the
+// waves' sums are added in wave order.
+template <typename CT, int D>
+__global__ __launch_bounds__(kThreads, 1) void bwd_dkcorr_split(BwdParams P) {
+  __shared__ __attribute__((aligned(16))) float st_s[kSplitWaves][2][kTileQ];
+  __shared__ __attribute__((aligned(16))) floatx4 dk_s[kSplitWaves][4 * kDTiles<D>][64];
+  const WorkItem item = xcd_work_item(P.kgroups, P.n, false, true, true);   // early keys (long walks) first
+  if (!item.valid) return;
+  const int64_t slice = item.slice;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
+  const int kb = item.idx, T = static_cast<int>(P.T), nq = (T + kTileQ - 1) / kTileQ;
+  const int key = kb * kTileK + l32;
+  const CT* qs = static_cast<const CT*>(P.q) + P.qv.slice(slice);
+  const CT* qgts = static_cast<const CT*>(P.qgt) + slice * D * P.t_pad;
+  const float* lse = P.lse + slice * P.T;
+  RowFrag<CT, D> kf;
+  global_row_frag<CT, D>(kf, static_cast<const CT*>(P.k) + P.kv.slice(slice), key, T - 1, P.kv.sr, h);
+  floatx16 dkc[kDTiles<D>];
+#pragma unroll
+  for (int t = 0; t < kDTiles<D>; ++t) dkc[t] = floatx16{};
+  struct F {
+    WalkFrags<CT, D, true> w;
+    float lse;
+  };
+  auto load = [&](F& f, int qt) {
+    global_row_frag<CT, D>(f.w.row, qs, qt * kTileQ + qsig(l32), T - 1, P.qv.sr, h);   // slot l32: row qsig(l32)
+    const int r = qt * kTileQ + l32;
+    f.lse = r < T ? lse[r] : INFINITY;
+#pragma unroll
+    for (int t = 0; t < kDTiles<D>; ++t)
+      global_t_frags<CT, D, true>(f.w.t[t], qgts + static_cast<int64_t>(qt) * kTileQ * D, 32 * t + l32, h);
+  };
+  int buf = 0;
+  auto step = [&](const F& f, int qt) {
+    st_s[wave][buf][l32] = f.lse;                  // within the wave: no barrier
+    const floatx16 sacc = mma_rows<CT, D>(f.w.row, kf, floatx16{});
+    float lz[16], p[16];
+    lds_read16(st_s[wave][buf] + 16 * h, lz);
+    buf ^= 1;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) p[i] = fast_exp2(fmaf(sacc[i], P.c, -lz[i]));
+    if (qt == kb) {
+      const int dk = l32 - 16 * h;                 // key - row(i) = dk - i on the diagonal tile
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (dk > i) p[i] = 0.f;
+    }
+#pragma unroll
+    for (int s = 0; s < kSlots<CT>; ++s) {
+      const auto bfr = acc_frag<CT>(p, s);
+#pragma unroll
+      for (int t = 0; t < kDTiles<D>; ++t) dkc[t] = Mma<CT>::mma(f.w.t[t][s], bfr, dkc[t]);
+    }
+  };
+  walk_tiles<kWalkAhead<CT, D>, F>(kb + wave, nq, load, step);
+#pragma unroll
+  for (int t = 0; t < kDTiles<D>; ++t)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      dk_s[wave][4 * t + j][lane] = floatx4{dkc[t][4 * j], dkc[t][4 * j + 1], dkc[t][4 * j + 2], dkc[t][4 * j + 3]};
+  __syncthreads();
+  if (key >= T) return;
+  const int64_t base = (slice * P.T + key) * D, out = P.gkv.slice(slice) + key * P.gkv.sr;
+#pragma unroll
+  for (int c = 0; c < kDTiles<D>; ++c) {
+    const int q = wave + kSplitWaves * c;          // chunk: head dims 32 (q / 4) + 8 (q % 4) + 4 h + [0, 4)
+    const int d = 32 * (q >> 2) + 8 * (q & 3) + 4 * h;
+    if (d < D) {
+      const floatx4 corr = (dk_s[0][q][lane] + dk_s[1][q][lane]) + (dk_s[2][q][lane] + dk_s[3][q][lane]);
+      const floatx4 dm = *reinterpret_cast<const floatx4*>(P.dkm + base + d);
+      store4_as(P.dk, out + d, P.gdt, (dm - corr) * P.scale);
+    }
   }
 }
 
@@ -1606,6 +1693,20 @@ int launch_backward(const BackwardArgs& a) {
   const bool rows_flat = P.qv.sr == D && P.kv.sr == D && P.vv.sr == D;
   return with_rows<is_production<BID, SHARE>() && D <= 128>(rows_flat, [&](auto flat_tag) -> int {
   constexpr bool kFlat = decltype(flat_tag)::value;
+  // the softmax-Jacobian correction of dk: split walks where they are few
+  auto dk_correction = [&](BwdParams K) {
+    if constexpr (is_production<BID, SHARE>() && D <= 128) {
+      if (split_walks<CT, D>(a.n, nkt)) {
+        K.kgroups = nkt;
+        DIL_TIMED("bwd_dkcorr", st,
+                  (bwd_dkcorr_split<CT, D><<<dim3(static_cast<unsigned>(xcd_grid(nkt * a.n))), kThreads, 0, st>>>(K)));
+        return;
+      }
+    }
+    K.kgroups = (nkt + 3) / 4;
+    const dim3 g(static_cast<unsigned>(xcd_grid(static_cast<int64_t>(K.kgroups) * key_split<CT, D>() * a.n)));
+    DIL_TIMED("bwd_dkcorr", st, (bwd_dkcorr<CT, D, BID, kFlat><<<g, kThreads, 0, st>>>(K)));
+  };
   if constexpr (std::is_same_v<CT, __bf16> && D == 64) {
     // the pass reads a slice's Q rows through one resource with 32-bit offsets
     const bool q_fits = a.T * P.qv.sr * static_cast<int64_t>(sizeof(CT)) < (int64_t{1} << 31);
@@ -1625,9 +1726,7 @@ int launch_backward(const BackwardArgs& a) {
                   (bwd_dq_reduce<D, kGhat><<<dim3(nq, ns), kThreads, 0, st>>>(dqp, ghp, ntiles, a.T, a.pk, qt, t_pad,
                                                                              a.dq, a.gqv, a.grad_dtype, P.scale, qgt, s0)));
       });
-      P.kgroups = (nkt + 3) / 4;
-      const dim3 gkey(static_cast<unsigned>(xcd_grid(static_cast<int64_t>(P.kgroups) * key_split<CT, D>() * a.n)));
-      DIL_TIMED("bwd_dkcorr", st, (bwd_dkcorr<CT, D, BID, kFlat><<<gkey, kThreads, 0, st>>>(P)));
+      dk_correction(P);
       return static_cast<int>(hipGetLastError());
     }
   }
@@ -1637,19 +1736,24 @@ int launch_backward(const BackwardArgs& a) {
   DIL_TIMED("bwd_key", st, (bwd_key<CT, D, BID, SHARE, kFlat><<<gkeys, kThreads, 0, st>>>(P)));
   constexpr bool kParked = query_parks<CT, D>() && is_production<BID, SHARE>();
   constexpr int kQW = kParked ? query_waves<CT, D>() : 4;     // row tiles (waves) per workgroup
-  {
-    const int kgroups_key = P.kgroups;
-    P.kgroups = (nkt + kQW - 1) / kQW;
-    const dim3 gq(static_cast<unsigned>(xcd_grid(static_cast<int64_t>(P.kgroups) * a.n)));
-    DIL_TIMED("bwd_query", st, (bwd_query<CT, D, BID, SHARE, kParked, kQW, kFlat><<<gq, 64 * kQW, 0, st>>>(P)));
-    P.kgroups = kgroups_key;
+  auto query = [&](auto waves) {
+    constexpr int W = decltype(waves)::value;
+    BwdParams Q = P;
+    Q.kgroups = (nkt + W - 1) / W;
+    const dim3 gq(static_cast<unsigned>(xcd_grid(static_cast<int64_t>(Q.kgroups) * a.n)));
+    DIL_TIMED("bwd_query", st, (bwd_query<CT, D, BID, SHARE, kParked, W, kFlat><<<gq, 64 * W, 0, st>>>(Q)));
+  };
+  const bool few = kQW == 8 && query_few(a.n, nkt);
+  if constexpr (kQW == 8) {
+    if (few) query(std::integral_constant<int, 4>{});
   }
+  if (!few) query(std::integral_constant<int, kQW>{});
   slice_batches(a.n, [&](int64_t s0, unsigned ns) {
     DIL_TIMED("prep", st,
               prep_ghat_q<CT, D><<<dim3(static_cast<unsigned>(t_pad / 32), ns), kThreads, 0, st>>>(
                   qt, P.ghat, a.T, t_pad, qgt, s0));
   });
-  DIL_TIMED("bwd_dkcorr", st, (bwd_dkcorr<CT, D, BID, kFlat><<<gkeys, kThreads, 0, st>>>(P)));
+  dk_correction(P);
   return static_cast<int>(hipGetLastError());
   });
 }

@@ -1058,6 +1058,15 @@ __global__ __launch_bounds__(kThreads) void fwd_out_reduce(const KoPart<KW>* __r
   }
 }
 
+}  // namespace
+}  // namespace dil
+
+#include "dil_split_impl.hpp"
+
+namespace dil {
+
+namespace {
+
 // ---------------------------------------------------------------------------
 // host side
 
@@ -1244,8 +1253,24 @@ int launch_forward(const ForwardArgs& a) {
   const dim3 grid(static_cast<unsigned>(xcd_grid(P.groups * a.n)));
   const int strided = with_rows<is_production<BID, SHARE>() && D <= 128>(flat, [&](auto flat_tag) -> int {
   constexpr bool kFlat = decltype(flat_tag)::value;
-  if (a.pk) DIL_TIMED("fwd_stats", st, (fwd_stats<CT, D, true, BID, kFlat><<<grid, kThreads, 0, st>>>(P)));
-  else DIL_TIMED("fwd_stats", st, (fwd_stats<CT, D, false, BID, kFlat><<<grid, kThreads, 0, st>>>(P)));
+  // Few tiles: their walks split over a workgroup's waves.  Not above 2048 keys
+  // where the key pass could run: there a slice's bits don't depend on how many
+  // slices are in the call.
+  constexpr bool kSplit = is_production<BID, SHARE>() && D <= 128;
+  const bool split = kSplit && (a.Tk <= 2048 || !could) && split_walks<CT, D>(a.n, P.nb);
+  const dim3 gsplit(static_cast<unsigned>(xcd_grid(P.nb * a.n)));   // one 32-row tile per workgroup
+  if constexpr (kSplit) {
+    if (split) {
+      FwdParams S = P;
+      S.groups = static_cast<int>(P.nb);
+      if (a.pk) DIL_TIMED("fwd_stats", st, (fwd_stats_split<CT, D, true><<<gsplit, kThreads, 0, st>>>(S)));
+      else DIL_TIMED("fwd_stats", st, (fwd_stats_split<CT, D, false><<<gsplit, kThreads, 0, st>>>(S)));
+    }
+  }
+  if (!split) {
+    if (a.pk) DIL_TIMED("fwd_stats", st, (fwd_stats<CT, D, true, BID, kFlat><<<grid, kThreads, 0, st>>>(P)));
+    else DIL_TIMED("fwd_stats", st, (fwd_stats<CT, D, false, BID, kFlat><<<grid, kThreads, 0, st>>>(P)));
+  }
   if constexpr (kKeyPassBuilt) {
     if (key_pass) {
       // one key pass forms the checkpoints, the totals and the share V
@@ -1293,10 +1318,28 @@ int launch_forward(const ForwardArgs& a) {
       return run(std::integral_constant<int, 16>{});
     }
   }
-  P.kgroups = static_cast<int>((a.Tk + 4 * kTileK - 1) / (4 * kTileK));
-  DIL_TIMED("fwd_demand", st,
-            (fwd_demand<CT, D, BID, kFlat><<<dim3(static_cast<unsigned>(xcd_grid(static_cast<int64_t>(P.kgroups) * a.n))),
-                                      kThreads, 0, st>>>(P)));
+  const bool split_demand = split && P.nb <= kSplitDemandBlocks;
+  if constexpr (kSplit) {
+    if (split_demand) {
+      FwdParams S = P;
+      S.kgroups = static_cast<int>((a.Tk + kTileK - 1) / kTileK);
+      const dim3 gk(static_cast<unsigned>(xcd_grid(static_cast<int64_t>(S.kgroups) * a.n)));
+      const size_t lds = static_cast<size_t>(P.nb) * kTileK * sizeof(float);
+      DIL_TIMED("fwd_demand", st, (fwd_demand_split<CT, D><<<gk, kThreads, lds, st>>>(S)));
+    }
+  }
+  if (!split_demand) {
+    P.kgroups = static_cast<int>((a.Tk + 4 * kTileK - 1) / (4 * kTileK));
+    const dim3 gk(static_cast<unsigned>(xcd_grid(static_cast<int64_t>(P.kgroups) * a.n)));
+    DIL_TIMED("fwd_demand", st, (fwd_demand<CT, D, BID, kFlat><<<gk, kThreads, 0, st>>>(P)));
+  }
+  if constexpr (kSplit) {
+    if (split) {
+      P.groups = static_cast<int>(P.nb);
+      DIL_TIMED("fwd_out", st, (fwd_out_split<CT, D><<<gsplit, kThreads, 0, st>>>(P)));
+      return static_cast<int>(hipGetLastError());
+    }
+  }
   DIL_TIMED("fwd_out", st, (fwd_out<CT, D, BID, SHARE, kFlat><<<grid, kThreads, 0, st>>>(P)));
   return static_cast<int>(hipGetLastError());
   });

@@ -1,0 +1,95 @@
+"""Calls with few 32-row tiles split each tile's walk over a workgroup's waves
+(split_walks, dil_walk.hpp), and fp32 / split operands take the dq pass in
+groups of 4 tiles instead of 8 (query_few).
+
+Forward, demand and gradients against the fp64 oracle at the edges of a tile
+and on both sides of each type's limit, with the bounds of the forward's and
+backward's own tests: fp32 operands 1e-4 max-abs, bf16 operands 2e-2 for the
+output and 5e-2 for the gradients.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from gpu_helpers import max_abs, needs_gpu
+from oracle import dilution_oracle as orc
+
+pytestmark = [pytest.mark.gpu, needs_gpu]
+
+# head dim, operand type, and the limit in tiles of that pair
+LIMITS = [(16, "bf16", 2048), (32, "bf16", 2048), (64, "bf16", 1280), (128, "bf16", 768), (64, "ieee", 2048),
+          (128, "ieee", 1024), (32, "tf32", 1024), (64, "tf32", 640), (128, "tf32", 640)]
+
+
+def _check(q, k, v, do, prec, slices):
+    """One call over all slices; the named slices against the oracle."""
+    from dilution import kernels
+
+    xs = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    out = kernels.dilution_attention(*xs, dot_precision=prec)
+    out.backward(do.cuda())
+    _, aux = kernels.dilution_attention_forward(*(x.detach() for x in xs), dot_precision=prec, return_aux=True)
+    b16 = prec == "bf16"
+    for s in slices:
+        one = [t[:, s:s + 1].double() for t in (q, k, v, do)]
+        want, _ = orc.grads_closed_form_f64(*(t.numpy() for t in one))
+        assert max_abs(out.detach()[:, s:s + 1], orc.attention_f64(*one[:3])) < (2e-2 if b16 else 1e-4)
+        for name, x, w in zip(("dq", "dk", "dv"), xs, want):
+            assert max_abs(x.grad[:, s:s + 1], torch.as_tensor(w)) < (5e-2 if b16 else 1e-4), (name, s)
+        scores = (one[0] @ one[1].transpose(-1, -2)) / q.shape[-1] ** 0.5
+        t = q.shape[-2]
+        total = scores.masked_fill(torch.ones(t, t, dtype=torch.bool).triu(1), float("-inf")).softmax(-1).sum(-2)
+        # the columns of p: fp32 exponentials (and, for bf16 operands, exact products of the given values)
+        assert max_abs(aux["committed_total"][:, s:s + 1], total) < 1e-5 * max(1.0, t ** 0.5)
+
+
+@pytest.mark.parametrize("dim,prec", [(d, p) for d, p, _ in LIMITS])
+@pytest.mark.parametrize("seq", [1, 31, 33, 129, 300])
+def test_tile_edges(dim, prec, seq):
+    dtype = torch.bfloat16 if prec == "bf16" else torch.float32
+    q, k, v, do = orc.make_inputs((1, 2, seq, dim), seed=seq + dim, qk_scale=0.5, with_dout=True, dtype=dtype)
+    _check(q, k, v, do, prec, (0, 1))
+
+
+@pytest.mark.parametrize("over", [0, 1])
+@pytest.mark.parametrize("dim,prec,limit", LIMITS)
+def test_both_sides_of_the_limit(dim, prec, limit, over):
+    """As many slices of 65 rows (3 tiles) as the limit takes, and one more."""
+    dtype = torch.bfloat16 if prec == "bf16" else torch.float32
+    heads = limit // 3 + over
+    q, k, v, do = orc.make_inputs((1, heads, 65, dim), seed=dim + over, qk_scale=0.5, with_dout=True, dtype=dtype)
+    _check(q, k, v, do, prec, (0, heads // 2, heads - 1))
+
+
+@pytest.mark.parametrize("prec", ["bf16", "ieee", "tf32"])
+@pytest.mark.parametrize("chunk", [37, 96])
+def test_prefill_chunks(prec, chunk):
+    """Chunks whose first row lies inside a tile, with demand carried in."""
+    from dilution import cache, kernels
+
+    dtype = torch.bfloat16 if prec == "bf16" else torch.float32
+    q, k, v = (t.cuda() for t in orc.make_inputs((1, 2, 300, 64), seed=chunk, qk_scale=0.5, dtype=dtype))
+    got, state = cache.begin_cache(q, k, v, capacity=300, chunk=chunk, dot_precision=prec)
+    assert max_abs(got, orc.attention_f64(q.cpu(), k.cpu(), v.cpu())) < (2e-2 if prec == "bf16" else 1e-4)
+    _, aux = kernels.dilution_attention_forward(q, k, v, dot_precision=prec, return_aux=True)
+    assert max_abs(state["committed"].reshape(1, 2, 300), aux["committed_total"].cpu()) < 2e-4
+
+
+def test_long_row_keeps_the_full_demand_walk():
+    """One slice of more row blocks than the split demand pass holds the sums of
+    (256) takes the statistics and the output split and the demand whole."""
+    from dilution import kernels
+
+    q, k, v = (t.cuda() for t in orc.make_inputs((1, 1, 8225, 32), seed=5, qk_scale=0.5, dtype=torch.float32))
+    out, aux = kernels.dilution_attention_forward(q, k, v, dot_precision="ieee", return_aux=True)
+    head, head_aux = kernels.dilution_attention_forward(*(x[:, :, :8192].contiguous() for x in (q, k, v)),
+                                                        dot_precision="ieee", return_aux=True)
+    # fp32 sums of the same terms in another order: 8192 demand terms below 1, in fp64
+    assert max_abs(out[:, :, :8192], head.cpu()) < 1e-5
+    p = (q[:, :, 8192:].double() @ k.double().transpose(-1, -2).contiguous()) / 32 ** 0.5
+    mask = torch.ones(8225, 8225, dtype=torch.bool, device="cuda").triu(1)[8192:]
+    tail = p.masked_fill(mask, float("-inf")).softmax(-1).sum(-2)
+    assert max_abs(aux["committed_total"][..., :8192].double() - head_aux["committed_total"].double(),
+                   tail[..., :8192].cpu()) < 1e-4
