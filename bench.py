@@ -111,9 +111,10 @@ ALGO_PRODUCTS = {
 }
 
 # Algorithmic bytes per key of each decode kernel (d = head_dim, bf16 cache):
-# dec_stats streams K; dec_apply streams V and reads + writes the demand.
+# dec_stats streams K; dec_apply streams V and reads + writes the demand; dec_one
+# (short contexts) does both.
 def decode_bytes_per_key(kernel: str, d: int) -> int:
-    return {"dec_stats": 2 * d, "dec_apply": 2 * d + 8}.get(kernel, 0)
+    return {"dec_stats": 2 * d, "dec_apply": 2 * d + 8, "dec_one": 4 * d + 8}.get(kernel, 0)
 
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic.json")

@@ -1123,7 +1123,7 @@ inline bool keyout_eligible(int64_t C, int64_t Tk, int64_t q0, int D, int prec, 
 // chain on a few CUs (2.05 or 1.33 us per 32-row tile), where fwd_demand's walks
 // are one score product and one exp2 sweep per tile (~0.5 us) and fwd_out spreads
 // over the rows.  Measured, us (fwd_demand + fwd_out, key pass + reduction):
-// B1 H4 T512 30 / 35, B3 H5 T1357 60 / 78, B1 H16 T2048 83 / 105, B4 H16 T2048
+// B1 H4 T512 30 / 35 (19 with split walks), B3 H5 T1357 60 / 78 (42), B1 H16 T2048 83 / 105 (66), B4 H16 T2048
 // 125 / 153, B4 H16 T1024 52 / 69, B16 H16 T256 26 / 31; beyond 2^17 tokens the
 // lead is gone (B8 H16 T2048 222 + 9 of V^T / 208).  Rows of more than 2048 keys
 // keep the key pass (its bits: a prefix has those of the whole sequence).
