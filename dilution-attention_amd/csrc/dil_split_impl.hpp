@@ -174,6 +174,10 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_demand_split(FwdParams P) {
   const float* rden = P.rden + slice * P.C;
   RowFrag<CT, D> kf;
   global_row_frag<CT, D>(kf, static_cast<const CT*>(P.k) + P.kv.slice(slice), key, Tk - 1, P.kv.sr, h);
+  // the carried demand, read by all 4 waves before the barrier: total may be the
+  // same memory (a prefill chunk advances its demand in place), and the last wave
+  // stores it after the barrier, whatever the other waves have reached
+  const float demand0 = (P.demand_in != nullptr && key < q0 && key_ok) ? P.demand_in[slice * P.din_sn + key] : 0.f;
   struct F {
     RowFrag<CT, D> row;
     float lse;
@@ -227,7 +231,7 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_demand_split(FwdParams P) {
   if (h == 0) tot_s[wave][l32] = run;
   __syncthreads();
   // demand entering the wave's first block: the carried demand and the earlier quarters
-  double at = (P.demand_in != nullptr && key < q0 && key_ok) ? static_cast<double>(P.demand_in[slice * P.din_sn + key]) : 0.0;
+  double at = static_cast<double>(demand0);
   for (int w = 0; w < wave; ++w) at += tot_s[w][l32];
   if (key_ok && h == 0) {
     float* ccol = P.carry + slice * P.nb * P.Tk + key;

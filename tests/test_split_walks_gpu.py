@@ -77,6 +77,45 @@ def test_prefill_chunks(prec, chunk):
     assert max_abs(state["committed"].reshape(1, 2, 300), aux["committed_total"].cpu()) < 2e-4
 
 
+@pytest.mark.parametrize("dim,prec,start,rows", [(64, "ieee", 1000, 300), (64, "tf32", 1000, 300), (64, "bf16", 1000, 300),
+                                                 (64, "bf16", 1024, 300), (32, "bf16", 37, 100), (128, "tf32", 70, 33)])
+def test_carried_demand_is_read_before_it_is_advanced(dim, prec, start, rows):
+    """A chunk's demand pass takes the carried demand from the memory that it
+    advances (committed): all 4 waves of a key tile have to read it before one
+    of them stores the new total.  Every checkpoint against fp64, the first one
+    (the carried demand itself) bit for bit, over 6 slices' key tiles at once.
+
+    Tolerance: the demand is below 4; its terms p <= 1 carry about 1e-5
+    relative (hardware exp2, scores rounded to fp32) and sum to less than 1 per
+    key beside the diagonal's few: 2e-5; outputs as in the tests above."""
+    from dilution import kernels
+
+    dtype = torch.bfloat16 if prec == "bf16" else torch.float32
+    g = torch.Generator(device="cuda").manual_seed(start + dim)
+    length, blocks = start + rows, (rows + 31) // 32
+    q = (0.5 * torch.randn(2, 3, rows, dim, device="cuda", generator=g)).to(dtype)
+    k, v = ((s * torch.randn(2, 3, length, dim, device="cuda", generator=g)).to(dtype) for s in (0.5, 1.0))
+    before = torch.zeros(2, 3, length + 9, device="cuda")
+    before[..., :start] = 3 * torch.rand(2, 3, start, device="cuda", generator=g)
+    kc, vc = (torch.cat([x, torch.zeros_like(x[:, :, :9])], dim=2) for x in (k, v))
+    scores = (q.double() @ k.double().transpose(-1, -2).contiguous()) / dim ** 0.5
+    future = torch.arange(length, device="cuda")[None, :] > start + torch.arange(rows, device="cuda")[:, None]
+    p = scores.masked_fill(future, float("-inf")).softmax(-1)
+    demand = before[:, :, None, :length].double() + p.cumsum(-2)          # after each row
+    share = p / (demand + 1e-9)
+    want = (share / (share.sum(-1, keepdim=True) + 1e-9)) @ v.double()
+    committed = before.clone()
+    out, aux = kernels.dilution_prefill_chunk(q, kc, vc, committed, start, dot_precision=prec, return_aux=True)
+    carry = aux["carry"].reshape(2, 3, blocks, length)
+    assert torch.equal(carry[:, :, 0, :start], before[..., :start])
+    for b in range(1, blocks):
+        end = min(length, start + 32 * (b + 1))
+        assert (carry[:, :, b, :end].double() - demand[:, :, 32 * b - 1, :end]).abs().max() < 2e-5, b
+    assert (committed[..., :length].double() - demand[:, :, -1]).abs().max() < 2e-5
+    assert torch.equal(committed[..., length:], before[..., length:])
+    assert (out.double() - want).abs().max() < (2e-2 if prec == "bf16" else 1e-4)
+
+
 def test_long_row_keeps_the_full_demand_walk():
     """One slice of more row blocks than the split demand pass holds the sums of
     (256) takes the statistics and the output split and the demand whole."""
