@@ -40,12 +40,16 @@ bool valid_rows(const dil_rows* r, int64_t batch, int64_t heads, int head_dim, i
 bool even_slices(const dil_rows* r, int64_t batch, int64_t heads) {
   return batch == 1 || heads == 1 || r->batch_stride == heads * r->head_stride;
 }
-dil::RowsView view_of(const dil_rows* r, int64_t batch, int64_t heads) {
+// The view of slices of `rows` rows.  A single row has no next one: its stride
+// (any, as torch leaves the strides of dimensions of size 1) is head_dim, so that
+// the forms built for rows head_dim apart take it.
+dil::RowsView view_of(const dil_rows* r, int64_t batch, int64_t heads, int64_t rows, int head_dim) {
+  const int64_t row_stride = rows == 1 ? head_dim : r->row_stride;
   if (even_slices(r, batch, heads))
-    return dil::flat_rows(heads == 1 ? r->batch_stride : r->head_stride, r->row_stride);
+    return dil::flat_rows(heads == 1 ? r->batch_stride : r->head_stride, row_stride);
   const uint32_t h = static_cast<uint32_t>(heads);
   const uint32_t magic = static_cast<uint32_t>(((uint64_t{1} << 32) + h - 1) / h);
-  return dil::RowsView{h, magic, r->batch_stride, r->head_stride, r->row_stride};
+  return dil::RowsView{h, magic, r->batch_stride, r->head_stride, row_stride};
 }
 // slices are counted in 32 bits by the views, and their batch found by one
 // multiplication (RowsView)
@@ -325,9 +329,9 @@ int dil_forward_rows(const dil_rows* q, const dil_rows* k, const dil_rows* v, in
   a.q = q->data;
   a.k = k->data;
   a.v = v->data;
-  a.qv = view_of(q, batch, heads);
-  a.kv = view_of(k, batch, heads);
-  a.vv = view_of(v, batch, heads);
+  a.qv = view_of(q, batch, heads, seq, head_dim);
+  a.kv = view_of(k, batch, heads, seq, head_dim);
+  a.vv = view_of(v, batch, heads, seq, head_dim);
   a.ov = dil::flat_rows(seq * head_dim, head_dim);
   fill_forward(a, batch * heads, seq, head_dim, dtype, precision, bid, share, shift, out, rmax, rden, ssum,
                carry, committed_total, pk, workspace, workspace_bytes, stream);
@@ -391,9 +395,9 @@ int dil_prefill_rows(const dil_rows* q_chunk, const void* k_cache, const void* v
     return dil::kErrShape;
   dil::ForwardArgs a{};
   a.q = q_chunk->data;
-  a.qv = view_of(q_chunk, batch, heads);
+  a.qv = view_of(q_chunk, batch, heads, chunk, head_dim);
   a.out = const_cast<void*>(out->data);
-  a.ov = view_of(out, batch, heads);
+  a.ov = view_of(out, batch, heads, chunk, head_dim);
   a.out_dtype = out_dtype;
   fill_prefill(a, k_cache, v_cache, batch * heads, chunk, start, capacity, head_dim, dtype, precision,
                committed, rmax, rden, ssum, carry, workspace, workspace_bytes, stream);
@@ -447,13 +451,13 @@ int dil_backward_rows(const dil_rows* q, const dil_rows* k, const dil_rows* v, c
   a.dq = const_cast<void*>(dq->data);
   a.dk = const_cast<void*>(dk->data);
   a.dv = const_cast<void*>(dv->data);
-  a.qv = view_of(q, batch, heads);
-  a.kv = view_of(k, batch, heads);
-  a.vv = view_of(v, batch, heads);
-  a.dov = view_of(dout, batch, heads);
-  a.gqv = view_of(dq, batch, heads);
-  a.gkv = view_of(dk, batch, heads);
-  a.gvv = view_of(dv, batch, heads);
+  a.qv = view_of(q, batch, heads, seq, head_dim);
+  a.kv = view_of(k, batch, heads, seq, head_dim);
+  a.vv = view_of(v, batch, heads, seq, head_dim);
+  a.dov = view_of(dout, batch, heads, seq, head_dim);
+  a.gqv = view_of(dq, batch, heads, seq, head_dim);
+  a.gkv = view_of(dk, batch, heads, seq, head_dim);
+  a.gvv = view_of(dv, batch, heads, seq, head_dim);
   fill_backward(a, out, rmax, rden, ssum, carry, pk, batch * heads, seq, head_dim, dtype, dout_dtype, grad_dtype,
                 precision, bid, share, shift, workspace, workspace_bytes, stream);
   return run_backward(a);

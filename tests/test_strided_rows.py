@@ -132,3 +132,34 @@ def test_prefill_on_views_writes_its_rows(chunk, prec, dtype, dim):
     assert y.dtype == dtype and y.is_contiguous()
     assert torch.equal(y, torch.cat(parts, dim=2).to(dtype))
     assert torch.equal(c["committed"], ref["committed"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", list(LAYOUTS))
+@pytest.mark.parametrize("shape,bid", [((1, 4, 1, 64), "softmax"), ((1, 4, 1, 64), "relu"), ((1, 2, 1, 32), "sigmoid"),
+                                       ((3, 1, 1, 64), "softplus"), ((1, 3, 1, 256), "softmax"), ((1, 1, 1, 16), "minshift")])
+def test_one_row_has_no_stride(layout, shape, bid):
+    """A call of one row takes views whatever torch says of the row's stride (a
+    (1, H, 1, D) view of a projection is contiguous to torch and keeps the
+    projection's): the variants and head_dim 256, which are built for rows
+    head_dim apart, among them."""
+    xs, dout = _inputs(shape, torch.bfloat16)
+    ops, kw = (kernels, {}) if bid == "softmax" else (kernels_bid, {"bid": bid})
+    want = _train(*xs, dout, "bf16", ops, **kw)
+    got = _train(*(LAYOUTS[layout](x) for x in xs), LAYOUTS[layout](dout), "bf16", ops, **kw)
+    for w, g in zip(want, got):
+        assert g.shape == w.shape and torch.equal(w, g)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim,bid_kw", [(256, {}), (64, {"bid": "relu"})])
+def test_one_row_prompts_and_chunks(dim, bid_kw):
+    """begin_cache on a projection's views: a prompt of one token, and a last
+    chunk of one row."""
+    for seq, chunk in ((1, None), (1, 8), (9, 8)):
+        if bid_kw and chunk:
+            continue
+        xs, _ = _inputs((1, 2, seq, dim), torch.bfloat16)
+        want, c0 = cache.begin_cache(*xs, capacity=12, chunk=chunk, **bid_kw)
+        got, c1 = cache.begin_cache(*(LAYOUTS["packed"](x) for x in xs), capacity=12, chunk=chunk, **bid_kw)
+        assert torch.equal(got, want) and torch.equal(c0["committed"], c1["committed"])
