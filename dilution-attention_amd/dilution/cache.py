@@ -84,13 +84,14 @@ def begin_cache(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, capacity: int
         return y.to(q.dtype), cache
     if chunk < 1:
         raise ValueError("chunk must be positive")
-    # every chunk writes its rows of y, in q's type
-    y = torch.empty(q.shape, device=q.device, dtype=q.dtype)
+    # every chunk writes its rows of y, in q's type where the kernels write it
+    # (fp64 queries get the fp32 outputs, converted)
+    y = torch.empty(q.shape, device=q.device, dtype=q.dtype if q.dtype in kernels._DTYPES else torch.float32)
     for start in range(0, seq, chunk):
         stop = min(start + chunk, seq)
         kernels.dilution_prefill_chunk(q[:, :, start:stop], cache["k"], cache["v"], cache["committed"], start,
                                        dot_precision=prec, _out=y[:, :, start:stop])
-    return y, cache
+    return y.to(q.dtype), cache
 
 
 def step_cache(q1: torch.Tensor, k1: torch.Tensor, v1: torch.Tensor, cache: dict, **bid_kw) -> torch.Tensor:

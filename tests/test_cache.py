@@ -124,3 +124,18 @@ def test_unwritten_cache_positions_are_never_read():
     assert torch.equal(y0, y1) and torch.equal(d0, d1)
     assert torch.equal(c0[..., :chunk + 1], c1[..., :chunk + 1])
     assert torch.isnan(c1[..., chunk + 1:]).all()
+
+
+@pytest.mark.gpu
+@needs_gpu
+@pytest.mark.parametrize("chunk", [None, 64])
+def test_fp64_queries_over_fp32_caches(chunk):
+    """Queries in a type that the kernels don't write (fp64 over fp32 K and V):
+    the fp32 outputs in the queries' type, in one call and in chunks."""
+    from dilution import cache as dc
+
+    q, k, v = (x.cuda() for x in orc.make_inputs((1, 2, 150, 64), seed=43))
+    want, c0 = dc.begin_cache(q, k, v, chunk=chunk)
+    got, c1 = dc.begin_cache(q.double(), k, v, chunk=chunk)
+    assert got.dtype == torch.float64
+    assert torch.equal(got, want.double()) and torch.equal(c0["committed"], c1["committed"])
