@@ -276,6 +276,8 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> backward(const at::Tensor& q, con
                                                         const py::tuple& variant, uintptr_t stream) {
   need_library();
   const int prec = precision_code(dot_precision);
+  // what a saved-tensor hook gave back, too
+  check_device({&q, &k, &v, &out, &rmax, &rden, &carry, &ssum, &pk, &dout});
   const Variant var = variant_of(variant);
   const int64_t batch = q.size(0), heads = q.size(1), seq = q.size(2), d = q.size(3), n = batch * heads;
   const at::ScalarType type = supported(at::promote_types(at::promote_types(q.scalar_type(), k.scalar_type()), v.scalar_type()));
@@ -425,6 +427,7 @@ at::Tensor rows_linear(const at::Tensor& x, const at::Tensor& w1, int mode, cons
     throw py::value_error("rows_linear: the normed modes need the norm weight g");
   if (mode == kSwiglu && !w2) throw py::value_error("rows_linear: the SwiGLU mode needs w2");
   if (mode == kResid && !resid) throw py::value_error("rows_linear: the residual mode needs resid");
+  check_device({&x});
   need_library();
   at::Tensor out;
   if (into) {
@@ -434,8 +437,7 @@ at::Tensor rows_linear(const at::Tensor& x, const at::Tensor& w1, int mode, cons
   } else {
     out = at::empty({rows, n}, x.options());
   }
-  c10::OptionalDeviceGuard guard;
-  if (x.is_cuda()) guard.reset_device(x.device());
+  c10::DeviceGuard guard(x.device());
   launch("dil_rows_linear", [&]() -> int {
     return api.rows_linear(x.data_ptr(), w1.data_ptr(), ptr(w2), ptr(g), ptr(resid), out.data_ptr(), rows, n, kk, mode, 1,
                            static_cast<float>(eps), reinterpret_cast<void*>(stream));
@@ -455,11 +457,11 @@ at::Tensor rows_linear_qkv(const at::Tensor& x, const at::Tensor& w, const at::T
     throw py::value_error("rows_linear_qkv: x, w and the caches disagree in shape");
   if (g.dim() != 1 || g.size(0) != kk)
     throw py::value_error("rows_linear_qkv: the norm weight must have shape (" + std::to_string(kk) + ",), got " + dims(g));
+  check_device({&x});
   need_library();
   if (pos_dev && (pos_dev->scalar_type() != at::kLong || pos_dev->numel() != 1 || pos_dev->device() != x.device()))
     throw py::value_error("a device position is a one-element int64 tensor on the inputs' device");
-  c10::OptionalDeviceGuard guard;
-  if (x.is_cuda()) guard.reset_device(x.device());
+  c10::DeviceGuard guard(x.device());
   at::Tensor q = at::empty({rows, heads * d}, x.options());
   launch("dil_rows_linear_qkv", [&]() -> int {
     return api.rows_linear_qkv(x.data_ptr(), w.data_ptr(), g.data_ptr(), q.data_ptr(), kc.data_ptr(), vc.data_ptr(), rows,

@@ -94,10 +94,12 @@ def rows_argmax(logits: torch.Tensor, limit: int | None = None, out: torch.Tenso
         out = torch.empty(rows, 1, device=logits.device, dtype=torch.int64)
     elif out.dtype != torch.int64 or out.numel() != rows or not out.is_contiguous() or out.device != logits.device:
         raise ValueError("out must be a contiguous int64 tensor of one element per row")
+    kernels._check_device(logits)
     status = _hip.lib().dil_rows_argmax(logits.data_ptr(), rows, logits.stride(0), limit, out.data_ptr(), 1,
                                         kernels._stream(logits.device))
     _hip.check(status, "dil_rows_argmax")
     return out
+
 
 @dataclass
 class LMConfig:

@@ -67,6 +67,25 @@ def test_rows_linear_rejects_mismatched_shapes():
         rows_linear_qkv(x, torch.zeros(512, 256, dtype=bf), g, 1e-5, kc, kc.clone(), 0)
 
 
+def test_projections_refuse_cpu_tensors():
+    """Operands of the right shapes and types that are not on the GPU are an
+    error on the host: a kernel would take their addresses for device memory."""
+    from dilution import kernels
+    from dilution.lm import rows_argmax, rows_linear, rows_linear_qkv
+
+    bf = torch.bfloat16
+    x, w, g = torch.zeros(4, 256, dtype=bf), torch.zeros(768, 256, dtype=bf), torch.ones(256, dtype=bf)
+    kc = torch.zeros(4, 2, 32, 128, dtype=bf)
+    q = torch.zeros(1, 2, 32, 64, dtype=bf)
+    rows, pk = torch.zeros(2, 32), torch.zeros(2, 32, 64)
+    for call in (lambda: rows_linear(x, w, 0), lambda: rows_linear_qkv(x, w, g, 1e-5, kc, kc.clone(), 0),
+                 lambda: rows_argmax(x),
+                 lambda: kernels._backward([q, q, q, q.float(), rows, rows, torch.zeros(2, 1, 32), rows, pk], q, "bf16",
+                                           kernels._PRODUCTION)):
+        with pytest.raises(RuntimeError, match="need tensors on the GPU"):
+            call()
+
+
 def test_config_validation():
     from dilution.lm import LMConfig
 
