@@ -340,8 +340,11 @@ __global__ __launch_bounds__(kDecThreads) void dec_one(OneSlice A, int64_t lengt
 // Chunk statistics: softmax bids (max, sum 2^(a - max)) in log2 units; ratio
 // bids (0 or the minimum of a for minshift, sum of the numerators) in natural
 // units; none for the elementwise bids.
-// ONE: a device-resident length that may be short: then the slice's first
-// workgroup does the whole step and the output launch has nothing to do.
+// ONE: a device-resident length that may be short: then one workgroup per slice
+// does the whole step and the output launch has nothing to do.  The launch's first
+// workgroups take the slices, one each, as they are dealt to the XCDs in turn: the
+// first workgroup of every slice would put them on one XCD for 8 chunks a slice (160
+// slices of 8000 keys, head_dim 128, of at most 20000, took 296 us so, and take 122).
 template <int D, int DT, int BID = BID_SOFTMAX, bool ONE = false>
 __global__ __launch_bounds__(kDecThreads) void dec_stats(
     const void* __restrict__ q1, int qdt, int64_t q_sn, const void* __restrict__ kc, int64_t kv_sn,
@@ -355,7 +358,8 @@ __global__ __launch_bounds__(kDecThreads) void dec_stats(
     extern __shared__ float one_s[];
     const int64_t live = live_length(dlen, length);
     if (live <= one_max_keys<D, DT>(nslices)) {
-      if (c == 0) one_slice<D, DT>(one, slice, static_cast<int>(live), one_s);
+      const unsigned block = blockIdx.y * gridDim.x + blockIdx.x;
+      if (block < gridDim.y) one_slice<D, DT>(one, slice0 + block, static_cast<int>(live), one_s);
       return;
     }
   }

@@ -103,3 +103,20 @@ def test_masked_affinities_and_zero_length():
         c = c0.clone()
         got = kernels.decode_step_device_length(q1, kc, vc, c, torch.tensor([0], device="cuda"), cap)
         assert (got == 0).all() and torch.equal(c, c0)
+
+
+@pytest.mark.parametrize("n,length,room", [(160, 2000, 20000), (9, 65, 70000), (3, 1, 300), (65, 1025, 4096), (257, 600, 33000)])
+def test_short_live_length_under_a_long_maximum(n, length, room):
+    """A graph's grid has a workgroup per slice and chunk of the longest length;
+    the first ones take a slice each when the live length is short: every slice
+    once, with the bits of the host length's step."""
+    from dilution import kernels
+
+    q1, kc, vc, c0 = _case(n, length, 32, torch.bfloat16, 3, length)
+    kc, vc = (torch.cat([x, x.new_zeros(1, n, room - x.shape[2], 32)], dim=2) for x in (kc, vc))
+    c0 = torch.cat([c0, c0.new_zeros(1, n, room - c0.shape[2])], dim=2)
+    c_host, c_dev = c0.clone(), c0.clone()
+    want = kernels.dilution_decode_step(q1, kc, vc, c_host, length)
+    _check(q1, kc, vc, c0, length, want, c_host)
+    got = kernels.decode_step_device_length(q1, kc, vc, c_dev, torch.tensor([length], device="cuda"), room)
+    assert torch.equal(got.reshape(-1), want.reshape(-1)) and torch.equal(c_dev, c_host)
