@@ -206,23 +206,34 @@ __device__ __forceinline__ int live_chunks(int64_t live, int64_t chunk) {
 // device-resident length, in the kernels.  One workgroup streams ~54 GB/s, so
 // with few slices the chunked step's many workgroups catch up at a few hundred
 // KB of K and V; from 160 slices on HBM bounds both and this form saves the
-// launches and the affinities' way through memory (up to 256 slices and from 512
-// on; in between the second round of workgroups is a partial one).  us per step
-// from memory, chunked -> here:
+// launches and the affinities' way through memory.  The workgroups run in rounds
+// of 256; where the last round leaves more than 3/16 of the rounds' places empty
+// the lead is gone above 768 KB (two rounds), 1 MB (three) or 2 MB a slice.  us
+// per step from memory, chunked -> here:
 //   bf16 64:  16 slices 512 keys 10.3 -> 6.4, 1000 11.2 -> 9.2, 2000 11.8 -> 13.9;
 //             64 slices 1000 12.6 -> 9.8, 2000 16.8 -> 15.1, 4000 21 -> 26;
 //             128 slices 2000 20 -> 18, 4000 31 -> 32; 192 slices 8000 76 -> 68;
 //             256 slices 1000 20 -> 14, 4000 54 -> 44, 16000 198 -> 170;
-//             288 slices 2000 41 -> 33, 4000 61 -> 62, 8000 113 -> 122; 1024 slices 4000 196 -> 173
-//   bf16 128: 16 slices 512 12 -> 9, 1000 13 -> 14; 64 slices 1000 15 -> 15
+//             288 slices 2000 41 -> 33, 4000 61 -> 62, 8000 113 -> 122; 512 slices 8000 186 -> 171;
+//             520 slices 2000 63 -> 54, 4000 107 -> 106, 8000 192 -> 211, 16000 371 -> 424;
+//             640 slices 8000 231 -> 224, 16000 452 -> 456; 832 slices 8000 299 -> 297, 16000 586 -> 605;
+//             1024 slices 4000 186 -> 174, 16000 722 -> 701; 2048 slices 16000 1433 -> 1408
+//   bf16 128: 16 slices 512 12 -> 9, 1000 13 -> 14; 64 slices 1000 15 -> 15; 520 slices 2000 112 -> 103,
+//             4000 198 -> 204, 16000 715 -> 843; 640 slices 16000 876 -> 898; 1024 slices 16000 1393 -> 1370
 //   fp32 64:  16 slices 512 13 -> 12, 1000 13 -> 18; 128 slices 512 16 -> 14, 1000 23 -> 25;
-//             256 slices 4000 107 -> 96
+//             256 slices 4000 107 -> 96; 520 slices 2000 131 -> 122, 4000 232 -> 248, 16000 864 -> 996;
+//             1024 slices 16000 1687 -> 1529
 constexpr int64_t kOneMaxKeys = 16384;                  // affinities a workgroup holds (64 KB of LDS)
 template <int D, int DT>
 __host__ __device__ inline int64_t one_max_keys(int64_t n) {
   constexpr int64_t kKeyBytes = 2 * D * (DT == DT_F32 ? 4 : 2);
-  if (n >= 512 || (n >= 160 && n <= 256)) return kOneMaxKeys;
-  if (n > 256) return (int64_t{768} << 10) / kKeyBytes;
+  if (n > 256) {
+    const int64_t places = (n + 255) / 256 * 256;
+    if (n >= 512 && 16 * n >= 13 * places) return kOneMaxKeys;
+    const int64_t keys = (n < 512 ? int64_t{768} : n < 768 ? int64_t{1024} : int64_t{2048}) * 1024 / kKeyBytes;
+    return keys < kOneMaxKeys ? keys : kOneMaxKeys;
+  }
+  if (n >= 160) return kOneMaxKeys;
   const int64_t keys = (DT == DT_F32 ? (256 + n) << 10 : (272 + 3 * n) << 10) / kKeyBytes;
   return keys < 4096 ? keys : 4096;
 }

@@ -120,3 +120,21 @@ def test_short_live_length_under_a_long_maximum(n, length, room):
     _check(q1, kc, vc, c0, length, want, c_host)
     got = kernels.decode_step_device_length(q1, kc, vc, c_dev, torch.tensor([length], device="cuda"), room)
     assert torch.equal(got.reshape(-1), want.reshape(-1)) and torch.equal(c_dev, c_host)
+
+
+@pytest.mark.parametrize("n,dim,dtype,limit", [(513, 64, torch.bfloat16, 4096), (623, 64, torch.float32, 2048),
+                                               (624, 16, torch.bfloat16, 16384), (770, 128, torch.bfloat16, 4096),
+                                               (1039, 32, torch.float16, 16384), (300, 16, torch.bfloat16, 12288)])
+def test_partial_last_round_of_workgroups(n, dim, dtype, limit):
+    """More than one round of 256 workgroups with a last one that leaves more
+    than 3/16 of their places empty: at most 768 KiB, 1 MiB (three rounds) or 2 MiB
+    of K and V a slice."""
+    from dilution import kernels
+
+    for length in (33, limit, limit + 1):
+        q1, kc, vc, c0 = _case(n, length, dim, dtype, 1, length)
+        c_host, c_dev = c0.clone(), c0.clone()
+        out = kernels.dilution_decode_step(q1, kc, vc, c_host, length)
+        _check(q1, kc, vc, c0, length, out, c_host)
+        got = kernels.decode_step_device_length(q1, kc, vc, c_dev, torch.tensor([length], device="cuda"), length + 1)
+        assert torch.equal(got.reshape(-1), out.reshape(-1)) and torch.equal(c_dev, c_host)
