@@ -1319,7 +1319,7 @@ int launch_forward(const ForwardArgs& a) {
       return run(std::integral_constant<int, 16>{});
     }
   }
-  const bool split_demand = split && P.nb <= kSplitDemandBlocks;
+  const bool split_demand = split && P.nb <= kSplitDemandBlocks && (a.q0 == 0 || split_demand_tiles<CT, D>(a.n, P.nb, a.Tk));
   if constexpr (kSplit) {
     if (split_demand) {
       FwdParams S = P;

@@ -152,6 +152,25 @@ __global__ __launch_bounds__(kThreads, 1) void fwd_stats_split(FwdParams P) {
 
 constexpr int kSplitDemandBlocks = 256;                // row blocks a workgroup keeps the sums of (32 KB)
 
+// Whether a chunk that starts past row 0 splits its demand walks.  The pass has a
+// workgroup per 32 keys, of which a chunk has more than row tiles (split_walks
+// counts those), each with a shorter walk: up to 3 blocks are one step per wave
+// and nothing is won.  fwd_demand, us, split / whole (key tiles x row blocks):
+//   bf16 64:  260x10 8.2 / 10.3, 656x10 11.3 / 11.6, 832x4 8.1 / 7.1, 2160x10 20 / 14, 16256x4 58 / 27
+//   bf16 32:  1040x10 8.6 / 11.3, 2624x10 15.4 / 16.1, 4160x10 20 / 16, 4304x19 27.2 / 27.4, 4032x32 30 / 35
+//   bf16 128: 269x19 15 / 17, 540x10 15 / 12, 1008x32 36 / 26
+//   fp32 64:  516x4 11.0 / 11.6, 656x10 22 / 22, 1016x4 16 / 12;  fp32 128: 269x19 36 / 52, 540x10 34 / 31
+//   split 64: 269x19 15 / 19, 540x10 15 / 13, 1008x32 36 / 28;  split 128: 260x10 16 / 16, 540x10 24 / 17
+template <typename CT, int D>
+inline bool split_demand_tiles(int64_t n, int64_t blocks, int64_t Tk) {
+  constexpr bool kNarrow = std::is_same_v<CT, __bf16> && D <= 32;      // the longer walks pay for more key tiles
+  constexpr int64_t kTiles = std::is_same_v<CT, float>     ? (D <= 64 ? 640 : 512)
+                             : std::is_same_v<CT, split32> ? (D <= 32 ? 512 : 320)
+                                                           : (D <= 32 ? 2048 : D <= 64 ? 640 : 384);
+  const int64_t limit = kNarrow && blocks >= 16 ? 2 * kTiles : kTiles;
+  return blocks > 3 && n * ((Tk + kTileK - 1) / kTileK) <= limit;
+}
+
 template <typename CT, int D>
 __global__ __launch_bounds__(kThreads, 1) void fwd_demand_split(FwdParams P) {
   extern __shared__ float csum_s[];                    // [row block][32 keys]: column sums of p

@@ -77,8 +77,40 @@ def test_prefill_chunks(prec, chunk):
     assert max_abs(state["committed"].reshape(1, 2, 300), aux["committed_total"].cpu()) < 2e-4
 
 
+def _check_chunk(heads, dim, prec, start, rows, slices):
+    """One prefill chunk over `heads` slices with demand carried in; the named
+    slices' checkpoints, totals and outputs against fp64."""
+    from dilution import kernels
+
+    dtype = torch.bfloat16 if prec == "bf16" else torch.float32
+    g = torch.Generator(device="cuda").manual_seed(start + dim)
+    length, blocks = start + rows, (rows + 31) // 32
+    q = (0.5 * torch.randn(1, heads, rows, dim, device="cuda", generator=g)).to(dtype)
+    k, v = ((s * torch.randn(1, heads, length, dim, device="cuda", generator=g)).to(dtype) for s in (0.5, 1.0))
+    before = torch.zeros(1, heads, length + 9, device="cuda")
+    before[..., :start] = 3 * torch.rand(1, heads, start, device="cuda", generator=g)
+    kc, vc = (torch.cat([x, torch.zeros_like(x[:, :, :1]).expand(-1, -1, 9, -1)], dim=2) for x in (k, v))
+    committed = before.clone()
+    out, aux = kernels.dilution_prefill_chunk(q, kc, vc, committed, start, dot_precision=prec, return_aux=True)
+    future = torch.arange(length, device="cuda")[None, :] > start + torch.arange(rows, device="cuda")[:, None]
+    for s in slices:
+        scores = (q[0, s].double() @ k[0, s].double().T.contiguous()) / dim ** 0.5
+        p = scores.masked_fill(future, float("-inf")).softmax(-1)
+        demand = before[0, s, :length].double() + p.cumsum(-2)            # after each row
+        share = p / (demand + 1e-9)
+        want = (share / (share.sum(-1, keepdim=True) + 1e-9)) @ v[0, s].double()
+        carry = aux["carry"].reshape(heads, blocks, length)[s]
+        assert torch.equal(carry[0, :start], before[0, s, :start]), s
+        for b in range(1, blocks):
+            end = min(length, start + 32 * (b + 1))
+            assert (carry[b, :end].double() - demand[32 * b - 1, :end]).abs().max() < 2e-5, (s, b)
+        assert (committed[0, s, :length].double() - demand[-1]).abs().max() < 2e-5, s
+        assert (out[0, s].double() - want).abs().max() < (2e-2 if prec == "bf16" else 1e-4), s
+    assert torch.equal(committed[..., length:], before[..., length:])
+
+
 @pytest.mark.parametrize("dim,prec,start,rows", [(64, "ieee", 1000, 300), (64, "tf32", 1000, 300), (64, "bf16", 1000, 300),
-                                                 (64, "bf16", 1024, 300), (32, "bf16", 37, 100), (128, "tf32", 70, 33)])
+                                                 (64, "bf16", 1024, 300), (32, "bf16", 37, 100), (128, "tf32", 70, 130)])
 def test_carried_demand_is_read_before_it_is_advanced(dim, prec, start, rows):
     """A chunk's demand pass takes the carried demand from the memory that it
     advances (committed): all 4 waves of a key tile have to read it before one
@@ -88,32 +120,21 @@ def test_carried_demand_is_read_before_it_is_advanced(dim, prec, start, rows):
     Tolerance: the demand is below 4; its terms p <= 1 carry about 1e-5
     relative (hardware exp2, scores rounded to fp32) and sum to less than 1 per
     key beside the diagonal's few: 2e-5; outputs as in the tests above."""
-    from dilution import kernels
+    _check_chunk(6, dim, prec, start, rows, range(6))
 
-    dtype = torch.bfloat16 if prec == "bf16" else torch.float32
-    g = torch.Generator(device="cuda").manual_seed(start + dim)
-    length, blocks = start + rows, (rows + 31) // 32
-    q = (0.5 * torch.randn(2, 3, rows, dim, device="cuda", generator=g)).to(dtype)
-    k, v = ((s * torch.randn(2, 3, length, dim, device="cuda", generator=g)).to(dtype) for s in (0.5, 1.0))
-    before = torch.zeros(2, 3, length + 9, device="cuda")
-    before[..., :start] = 3 * torch.rand(2, 3, start, device="cuda", generator=g)
-    kc, vc = (torch.cat([x, torch.zeros_like(x[:, :, :9])], dim=2) for x in (k, v))
-    scores = (q.double() @ k.double().transpose(-1, -2).contiguous()) / dim ** 0.5
-    future = torch.arange(length, device="cuda")[None, :] > start + torch.arange(rows, device="cuda")[:, None]
-    p = scores.masked_fill(future, float("-inf")).softmax(-1)
-    demand = before[:, :, None, :length].double() + p.cumsum(-2)          # after each row
-    share = p / (demand + 1e-9)
-    want = (share / (share.sum(-1, keepdim=True) + 1e-9)) @ v.double()
-    committed = before.clone()
-    out, aux = kernels.dilution_prefill_chunk(q, kc, vc, committed, start, dot_precision=prec, return_aux=True)
-    carry = aux["carry"].reshape(2, 3, blocks, length)
-    assert torch.equal(carry[:, :, 0, :start], before[..., :start])
-    for b in range(1, blocks):
-        end = min(length, start + 32 * (b + 1))
-        assert (carry[:, :, b, :end].double() - demand[:, :, 32 * b - 1, :end]).abs().max() < 2e-5, b
-    assert (committed[..., :length].double() - demand[:, :, -1]).abs().max() < 2e-5
-    assert torch.equal(committed[..., length:], before[..., length:])
-    assert (out.double() - want).abs().max() < (2e-2 if prec == "bf16" else 1e-4)
+
+@pytest.mark.parametrize("over", [0, 1])
+@pytest.mark.parametrize("dim,prec,limit", [(16, "bf16", 2048), (64, "bf16", 640), (128, "bf16", 384), (64, "ieee", 640),
+                                            (128, "ieee", 512), (32, "tf32", 512), (64, "tf32", 320)])
+def test_both_sides_of_the_key_tile_limit(dim, prec, limit, over):
+    """A chunk past row 0 counts key tiles for its demand pass: as many slices
+    of 8 key tiles (5 row blocks) as the limit takes, and one more; and chunks of
+    3 and 4 row blocks."""
+    heads = limit // 8 + over
+    _check_chunk(heads, dim, prec, 97, 147, (0, heads // 2, heads - 1))
+    _check_chunk(2, dim, prec, 130, 96 + over, (0, 1))
+    if (dim, prec) == (16, "bf16"):                            # 16 row blocks or more: twice the key tiles
+        _check_chunk(128 + over, dim, prec, 500, 512, (0, 127))
 
 
 def test_long_row_keeps_the_full_demand_walk():
