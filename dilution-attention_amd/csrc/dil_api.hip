@@ -111,7 +111,7 @@ void fill_forward(dil::ForwardArgs& a, int64_t n, int64_t seq, int head_dim, int
                   int share, float shift, float* out, float* rmax, float* rden, float* ssum, float* carry,
                   float* committed_total, float* pk, void* workspace, int64_t workspace_bytes, void* stream) {
   a.key_pass = dil::forward_key_pass_requested();
-  a.n = n;
+  a.n = a.call_n = n;
   a.C = seq;
   a.Tk = seq;
   a.q0 = 0;
@@ -144,7 +144,7 @@ void fill_prefill(dil::ForwardArgs& a, const void* k_cache, const void* v_cache,
   a.k = k_cache;
   a.v = v_cache;
   a.kv = a.vv = dil::flat_rows(capacity * head_dim, head_dim);
-  a.n = n;
+  a.n = a.call_n = n;
   a.C = chunk;
   a.Tk = start + chunk;
   a.q0 = start;
@@ -316,13 +316,14 @@ int dil_forward_variant(const void* q, const void* k, const void* v, int64_t n, 
   return run_forward(a);
 }
 
-int dil_forward_rows(const dil_rows* q, const dil_rows* k, const dil_rows* v, int64_t batch, int64_t heads,
-                     int64_t seq, int head_dim, int dtype, int precision, int bid, int share, float shift,
-                     float* out, float* rmax, float* rden, float* ssum, float* carry, float* committed_total,
-                     float* pk, void* workspace, int64_t workspace_bytes, void* stream) {
+int dil_forward_rows_group(const dil_rows* q, const dil_rows* k, const dil_rows* v, int64_t batch, int64_t heads,
+                           int64_t call_slices, int64_t seq, int head_dim, int dtype, int precision, int bid,
+                           int share, float shift, float* out, float* rmax, float* rden, float* ssum,
+                           float* carry, float* committed_total, float* pk, void* workspace,
+                           int64_t workspace_bytes, void* stream) {
   if (!valid_head_dim(head_dim, precision)) return dil::kErrHeadDim;
   if (!valid_dtype(dtype)) return dil::kErrDtype;
-  if (!valid_slices(batch, heads) || seq < 1) return dil::kErrShape;
+  if (!valid_slices(batch, heads) || call_slices < batch * heads || seq < 1) return dil::kErrShape;
   for (const dil_rows* r : {q, k, v})
     if (!valid_rows(r, batch, heads, head_dim, dtype)) return dil::kErrShape;
   dil::ForwardArgs a{};
@@ -335,7 +336,17 @@ int dil_forward_rows(const dil_rows* q, const dil_rows* k, const dil_rows* v, in
   a.ov = dil::flat_rows(seq * head_dim, head_dim);
   fill_forward(a, batch * heads, seq, head_dim, dtype, precision, bid, share, shift, out, rmax, rden, ssum,
                carry, committed_total, pk, workspace, workspace_bytes, stream);
+  a.call_n = call_slices;
   return run_forward(a);
+}
+
+int dil_forward_rows(const dil_rows* q, const dil_rows* k, const dil_rows* v, int64_t batch, int64_t heads,
+                     int64_t seq, int head_dim, int dtype, int precision, int bid, int share, float shift,
+                     float* out, float* rmax, float* rden, float* ssum, float* carry, float* committed_total,
+                     float* pk, void* workspace, int64_t workspace_bytes, void* stream) {
+  return dil_forward_rows_group(q, k, v, batch, heads, batch * heads, seq, head_dim, dtype, precision, bid, share,
+                                shift, out, rmax, rden, ssum, carry, committed_total, pk, workspace,
+                                workspace_bytes, stream);
 }
 
 int dil_forward(const void* q, const void* k, const void* v, int64_t n, int64_t seq,

@@ -1262,7 +1262,7 @@ int launch_forward(const ForwardArgs& a) {
   // where the key pass could run: there a slice's bits don't depend on how many
   // slices are in the call.
   constexpr bool kSplit = is_production<BID, SHARE>() && D <= 128;
-  const bool split = kSplit && (a.Tk <= 2048 || !could) && split_walks<CT, D>(a.n, P.nb);
+  const bool split = kSplit && (a.Tk <= 2048 || !could) && split_walks<CT, D>(a.call_n, P.nb);
   const dim3 gsplit(static_cast<unsigned>(xcd_grid(P.nb * a.n)));   // one 32-row tile per workgroup
   if constexpr (kSplit) {
     if (split) {

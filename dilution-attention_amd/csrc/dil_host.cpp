@@ -35,7 +35,7 @@ struct Api {
   decltype(&dil_status_string) status_string = nullptr;
   decltype(&dil_forward_key_pass) forward_key_pass = nullptr;
   decltype(&dil_forward_workspace_bytes) forward_workspace_bytes = nullptr;
-  decltype(&dil_forward_rows) forward_rows = nullptr;
+  decltype(&dil_forward_rows_group) forward_rows_group = nullptr;
   decltype(&dil_backward_workspace_bytes) backward_workspace_bytes = nullptr;
   decltype(&dil_backward_rows) backward_rows = nullptr;
   decltype(&dil_prefill_workspace_bytes) prefill_workspace_bytes = nullptr;
@@ -57,7 +57,7 @@ void bind(const py::dict& a) {
   take(api.status_string, a, "dil_status_string");
   take(api.forward_key_pass, a, "dil_forward_key_pass");
   take(api.forward_workspace_bytes, a, "dil_forward_workspace_bytes");
-  take(api.forward_rows, a, "dil_forward_rows");
+  take(api.forward_rows_group, a, "dil_forward_rows_group");
   take(api.backward_workspace_bytes, a, "dil_backward_workspace_bytes");
   take(api.backward_rows, a, "dil_backward_rows");
   take(api.prefill_workspace_bytes, a, "dil_prefill_workspace_bytes");
@@ -253,8 +253,8 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, Maybe, Ma
         advance(rk, ks);
         advance(rv, vs);
       }
-      const int status = api.forward_rows(
-          &rq, &rk, &rv, rows < n ? c : sd.first, sd.second, seq, static_cast<int>(d), tc, prec, var.bid, var.share,
+      const int status = api.forward_rows_group(
+          &rq, &rk, &rv, rows < n ? c : sd.first, sd.second, n, seq, static_cast<int>(d), tc, prec, var.bid, var.share,
           var.shift, f32(out) + a * seq * d, f32(rmax) + a * seq, f32(rden) + a * seq, f32(ssum) + a * seq,
           carry ? f32(*carry) : nullptr, f32(total) + a * seq, pk ? f32(*pk) + a * seq * d : nullptr, ws.data_ptr(),
           ws.numel(), reinterpret_cast<void*>(stream));

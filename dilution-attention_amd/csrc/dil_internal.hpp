@@ -138,6 +138,7 @@ struct ForwardArgs {
   const void* v;
   RowsView vv;
   int64_t n, C, Tk, q0;
+  int64_t call_n;        // slices of the whole call that these are a group of (n: all): picks the forms
   int head_dim, dtype, prec;   // precision code: 0 fp32, 1 split (tf32), 2 bf16 MFMA operands
   void* out;             // C rows per slice, in out_dtype
   RowsView ov;

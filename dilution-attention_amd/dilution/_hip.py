@@ -54,6 +54,9 @@ SIGNATURES = {
     "dil_forward_rows": (_c_int, [_rows_p, _rows_p, _rows_p, _c_int64, _c_int64, _c_int64, _c_int, _c_int,
                                   _c_int, _c_int, _c_int, ctypes.c_float,
                                   _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_int64, _vp]),
+    "dil_forward_rows_group": (_c_int, [_rows_p, _rows_p, _rows_p, _c_int64, _c_int64, _c_int64, _c_int64, _c_int,
+                                        _c_int, _c_int, _c_int, _c_int, ctypes.c_float,
+                                        _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_int64, _vp]),
     "dil_backward_rows": (_c_int, [_rows_p, _rows_p, _rows_p, _rows_p, _vp, _vp, _vp, _vp, _vp, _vp,
                                    _c_int64, _c_int64, _c_int64, _c_int, _c_int, _c_int, _c_int, _c_int,
                                    _c_int, _c_int, ctypes.c_float, _rows_p, _rows_p, _rows_p, _vp,

@@ -267,6 +267,17 @@ int dil_forward_rows(const dil_rows* q, const dil_rows* k, const dil_rows* v, in
                      int64_t seq, int head_dim, int dtype, int precision, int bid, int share, float shift,
                      float* out, float* rmax, float* rden, float* ssum, float* carry, float* committed_total,
                      float* pk, void* workspace, int64_t workspace_bytes, void* stream);
+/*
+ * A group of the slices of a larger call (call_slices >= batch * heads of them),
+ * for a caller that works in groups to bound its checkpoint scratch: the kernels'
+ * forms are picked by the whole call's size, so that every slice gets the bits
+ * that one call over all of them gives.
+ */
+int dil_forward_rows_group(const dil_rows* q, const dil_rows* k, const dil_rows* v, int64_t batch, int64_t heads,
+                           int64_t call_slices, int64_t seq, int head_dim, int dtype, int precision, int bid,
+                           int share, float shift, float* out, float* rmax, float* rden, float* ssum,
+                           float* carry, float* committed_total, float* pk, void* workspace,
+                           int64_t workspace_bytes, void* stream);
 int dil_backward_rows(const dil_rows* q, const dil_rows* k, const dil_rows* v, const dil_rows* dout,
                       const float* out, const float* rmax, const float* rden, const float* ssum,
                       const float* carry, const float* pk, int64_t batch, int64_t heads, int64_t seq,

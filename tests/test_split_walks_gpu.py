@@ -137,6 +137,24 @@ def test_both_sides_of_the_key_tile_limit(dim, prec, limit, over):
         _check_chunk(128 + over, dim, prec, 500, 512, (0, 127))
 
 
+@pytest.mark.parametrize("dim,prec,limit", [(64, "ieee", 2048), (64, "tf32", 640), (128, "bf16", 768), (32, "bf16", 2048)])
+def test_groups_have_the_bits_of_the_whole_call(dim, prec, limit):
+    """A call without aux whose checkpoint scratch is over its budget runs its
+    slices in groups: a call just above the limit in groups below it, and one
+    below the limit."""
+    from dilution import kernels
+
+    dtype = torch.bfloat16 if prec == "bf16" else torch.float32
+    g = torch.Generator(device="cuda").manual_seed(dim)
+    for heads in (limit // 3 + 1, limit // 3 - 1):                        # 3 row tiles per slice
+        q, k, v = (torch.randn(1, heads, 90, dim, device="cuda", generator=g).to(dtype) for _ in range(3))
+        whole = kernels.dilution_attention_forward(q, k, v, dot_precision=prec)
+        for rows in (heads // 2, heads - 1, 1 if heads < 300 else heads // 7):
+            budget = (rows + 0.5) * 3 * 90 * 4 / 2 ** 30
+            assert torch.equal(whole, kernels.dilution_attention_forward(q, k, v, dot_precision=prec,
+                                                                         scratch_budget_gib=budget)), (heads, rows)
+
+
 def test_long_row_keeps_the_full_demand_walk():
     """One slice of more row blocks than the split demand pass holds the sums of
     (256) takes the statistics and the output split and the demand whole."""
