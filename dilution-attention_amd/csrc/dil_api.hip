@@ -68,7 +68,7 @@ int run_forward(const dil::ForwardArgs& a) {
                static_cast<const void*>(a.rden), static_cast<const void*>(a.ssum),
                static_cast<const void*>(a.total), static_cast<const void*>(a.workspace)))
     return dil::kErrShape;
-  if (a.workspace_bytes < dil::forward_workspace_bytes(a.n, a.C, a.Tk, a.head_dim, a.dtype, a.prec,
+  if (a.workspace_bytes < dil::forward_workspace_least(a.n, a.C, a.Tk, a.head_dim, a.dtype, a.prec,
                                                        a.pk != nullptr, a.key_pass))
     return dil::kErrWorkspace;
   return dil::forward(a);

@@ -21,7 +21,13 @@ int dispatch_forward(const ForwardArgs& a) {
 
 int64_t forward_workspace_bytes(int64_t n, int64_t C, int64_t Tk, int head_dim, int dtype, int prec,
                                 int want_pk, bool key_pass) {
-  return static_cast<int64_t>(fwd_layout(n, C, Tk, head_dim, dtype, prec, want_pk, key_pass).total);
+  return static_cast<int64_t>(
+      fwd_layout(n, C, Tk, head_dim, dtype, prec, want_pk, key_pass, keyout_waves(n, C, Tk, head_dim)).total);
+}
+
+int64_t forward_workspace_least(int64_t n, int64_t C, int64_t Tk, int head_dim, int dtype, int prec,
+                                int want_pk, bool key_pass) {
+  return static_cast<int64_t>(fwd_layout(n, C, Tk, head_dim, dtype, prec, want_pk, key_pass, kKeyoutWaves).total);
 }
 
 bool forward_takes_key_pass(int64_t C, int64_t Tk, int64_t q0, int head_dim, int prec, const Variant& var,

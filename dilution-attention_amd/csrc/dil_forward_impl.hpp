@@ -1151,8 +1151,9 @@ struct FwdWorkspace {
   size_t vt, kt, qc, kc, op, rp, carry, total;
 };
 
+// kw: the waves per key group of the key pass, where the call takes it
 FwdWorkspace fwd_layout(int64_t n, int64_t C, int64_t Tk, int D, int dtype, int prec, int want_pk,
-                        bool key_pass) {
+                        bool key_pass, int kw) {
   const size_t ct = prec == 2 ? 2 : 4;
   const bool convert = dtype != native_dtype(prec);
   FwdWorkspace w{};
@@ -1171,7 +1172,6 @@ FwdWorkspace fwd_layout(int64_t n, int64_t C, int64_t Tk, int D, int dtype, int 
     // the three-pass forward's checkpoints, for a caller that keeps none
     w.total = w.carry + align_up(static_cast<size_t>(4 * n * ((C + kTileQ - 1) / kTileQ) * Tk));
   } else if (keyout_eligible(C, Tk, Tk - C, D, prec, key_pass)) {
-    const int kw = keyout_waves(n, C, Tk, D);
     const int64_t tiles = keyout_batch(kw, n, C, Tk, D) * keyout_tiles(kw, C, Tk);
     w.rp = w.op + align_up(static_cast<size_t>(tiles * D * kTileQ * keyout_part_size(kw)));
     w.total = w.rp + align_up(static_cast<size_t>(tiles * kTileQ * 4));
@@ -1179,9 +1179,22 @@ FwdWorkspace fwd_layout(int64_t n, int64_t C, int64_t Tk, int D, int dtype, int 
   return w;
 }
 
+// The waves per key group of a call in this workspace: groups of 256 keys hold
+// four times the partials, so a workspace that was sized for more slices (which
+// take groups of 512) may not hold them.  The bits are the same.
+inline int keyout_waves_in(const ForwardArgs& a, int prec) {
+  const int kw = keyout_waves(a.n, a.C, a.Tk, a.head_dim);
+  const auto bytes = [&](int waves) {
+    return static_cast<int64_t>(
+        fwd_layout(a.n, a.C, a.Tk, a.head_dim, a.dtype, prec, a.pk != nullptr, a.key_pass, waves).total);
+  };
+  return kw == kKeyoutWaves || a.workspace_bytes >= bytes(kw) ? kw : kKeyoutWaves;
+}
+
 template <typename CT, int D, int BID = BID_SOFTMAX, int SHARE = SHARE_INCL>
 int launch_forward(const ForwardArgs& a) {
-  const FwdWorkspace w = fwd_layout(a.n, a.C, a.Tk, D, a.dtype, kOperandPrec<CT>, a.pk != nullptr, a.key_pass);
+  const int kw = keyout_waves_in(a, kOperandPrec<CT>);
+  const FwdWorkspace w = fwd_layout(a.n, a.C, a.Tk, D, a.dtype, kOperandPrec<CT>, a.pk != nullptr, a.key_pass, kw);
   char* ws = static_cast<char*>(a.workspace);
   hipStream_t st = static_cast<hipStream_t>(a.stream);
   const bool convert = a.dtype != kNativeDtype<CT>;
@@ -1280,8 +1293,8 @@ int launch_forward(const ForwardArgs& a) {
     if (key_pass) {
       // one key pass forms the checkpoints, the totals and the share V
       // partials; the reduction finishes out and ssum
-      auto run = [&](auto kw) -> int {
-      constexpr int KW = decltype(kw)::value;
+      auto run = [&](auto waves) -> int {
+      constexpr int KW = decltype(waves)::value;
       using KG = KeyGroups<KW>;
       KoPart<KW>* op = reinterpret_cast<KoPart<KW>*>(ws + w.op);
       float* rp = reinterpret_cast<float*>(ws + w.rp);
@@ -1319,7 +1332,7 @@ int launch_forward(const ForwardArgs& a) {
       }
       return static_cast<int>(hipGetLastError());
       };
-      if (keyout_waves(a.n, a.C, a.Tk, D) == 8) return run(std::integral_constant<int, 8>{});
+      if (kw == 8) return run(std::integral_constant<int, 8>{});
       return run(std::integral_constant<int, 16>{});
     }
   }

@@ -171,6 +171,9 @@ inline bool forward_key_pass_requested() {
 
 int64_t forward_workspace_bytes(int64_t n, int64_t C, int64_t Tk, int head_dim, int dtype, int prec,
                                 int want_pk, bool key_pass);
+// The least a call runs in (forward_workspace_bytes: the most it has use for)
+int64_t forward_workspace_least(int64_t n, int64_t C, int64_t Tk, int head_dim, int dtype, int prec,
+                                int want_pk, bool key_pass);
 // Whether a forward over rows [q0, q0 + C) against keys [0, Tk) takes the
 // key-parallel output pass, whose demand checkpoints are an output only (the
 // caller may then pass no carry array); the three-pass forward reads them.

@@ -32,6 +32,10 @@
  *   - The key-parallel forward's workspace holds at most 24 GiB of output
  *     partials; a call whose slices need more runs over them in batches, so
  *     the forward workspace stays bounded at any batch size.
+ *   - The forward's and the prefill's workspace queries are not monotone in the
+ *     slice count: a smaller call may be quicker with up to 1 GiB of partials
+ *     that a larger one has no use for.  A workspace sized for more slices of
+ *     the same rows (up to the 24 GiB) also runs fewer, with the same results.
  *   - Return value: 0 on success, a positive hipError_t from the launch, or a
  *     negative argument error (see dil_status_string).  A NULL pointer where
  *     an argument is required is an argument error (-4); only `pk` of

@@ -104,3 +104,26 @@ def test_inference_has_the_bits_of_training(heads, seq):
     assert torch.equal(train.detach(), kernels.dilution_attention(*xs, dot_precision="bf16"))
     out, aux = kernels.dilution_attention_forward(*xs, dot_precision="bf16", return_aux=True)
     assert torch.equal(out, train.detach())
+
+
+@pytest.mark.parametrize("seq,few,many", [(4096, 32, 48), (4096, 3, 200), (2048, 65, 96), (2048, 64, 96), (2048, 8, 65), (300, 40, 500)])
+def test_a_workspace_for_more_slices_runs_fewer(seq, few, many):
+    """A C caller that sizes its workspace once, for its largest batch: smaller
+    calls run in it with the bits of a call in their own (larger) one."""
+    from dilution import _hip
+
+    lib = _hip.lib()
+    g = torch.Generator(device="cuda").manual_seed(seq)
+    q, k, v = (torch.randn(few, seq, 64, device="cuda", generator=g).to(torch.bfloat16) for _ in range(3))
+    sizes = [lib.dil_forward_workspace_bytes(n, seq, 64, 1, 2, 0) for n in (few, many)]
+    assert lib.dil_prefill_workspace_bytes(many, seq, 0, 64, 1, 2) == sizes[1]
+    got = []
+    for size in sizes:
+        out = torch.empty(few, seq, 64, device="cuda")
+        stats = [torch.empty(few, seq, device="cuda") for _ in range(4)]
+        ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+        _hip.check(lib.dil_forward(q.data_ptr(), k.data_ptr(), v.data_ptr(), few, seq, 64, 1, 2, out.data_ptr(),
+                                   *(s.data_ptr() for s in stats[:3]), None, stats[3].data_ptr(), None, ws.data_ptr(),
+                                   size, torch.cuda.current_stream().cuda_stream), "dil_forward")
+        got.append([out, *stats])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
