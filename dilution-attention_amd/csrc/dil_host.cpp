@@ -47,6 +47,7 @@ struct Api {
 };
 Api api;
 bool bound = false;
+std::string why_unbound = "not loaded";
 
 template <typename F>
 void take(F& f, const py::dict& addresses, const char* name) {
@@ -70,7 +71,7 @@ void bind(const py::dict& a) {
 }
 
 void need_library() {
-  if (!bound) throw std::runtime_error("dilution HIP kernels are not available");
+  if (!bound) throw std::runtime_error("dilution HIP kernels are not available: " + why_unbound);
 }
 
 void check_status(int status, const char* what) {
@@ -484,6 +485,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     }
   });
   m.def("bind", &bind, "take the library's entry points, {name: address}");
+  m.def("unavailable", [](const std::string& why) { why_unbound = why; }, "the reason a call gives without bind");
   m.def("strided_rows", &strided_rows);
   m.def("slice_dims", &slice_dims);
   m.def("empty_as", &empty_as);

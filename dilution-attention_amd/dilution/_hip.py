@@ -105,19 +105,29 @@ def _load():
     except OSError as exc:  # missing ROCm runtime, wrong arch, ...
         _load_error = f"cannot load {LIB_PATH}: {exc}"
         return None
+    missing = [name for name in SIGNATURES if not hasattr(lib, name)]
+    if "dil_abi_version" not in missing and lib.dil_abi_version() != ABI_VERSION:
+        _load_error = f"{LIB_PATH} has ABI {lib.dil_abi_version()}, expected {ABI_VERSION}"
+        return None
+    if missing:   # an older build of this ABI, or another library
+        _load_error = f"{LIB_PATH} lacks {', '.join(missing)}"
+        return None
     for name, (res, args) in SIGNATURES.items():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
-    if lib.dil_abi_version() != ABI_VERSION:
-        _load_error = f"{LIB_PATH} has ABI {lib.dil_abi_version()}, expected {ABI_VERSION}"
-        return None
     _lib = lib
     return lib
 
 
 def available() -> bool:
     return _load() is not None
+
+
+def load_error() -> str | None:
+    """Why the library is not available (None while it is)."""
+    _load()
+    return _load_error
 
 
 def lib():

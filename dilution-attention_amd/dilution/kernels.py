@@ -34,8 +34,11 @@ try:
     from . import _host
 except ImportError as exc:              # not built, or built for another torch
     _host, _host_error = None, str(exc)
-if _host is not None and _hip.available():
-    _host.bind(_hip.addresses())
+if _host is not None:
+    if _hip.available():
+        _host.bind(_hip.addresses())
+    else:
+        _host.unavailable(_hip.load_error())
 
 HAS_HIP = _hip.available() and _host is not None
 """True when libdilution_hip.so and the native host module are built and

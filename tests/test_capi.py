@@ -393,3 +393,33 @@ def test_integration_loader_re_exports_the_module(monkeypatch):
     finally:
         for mod in [m for m in sys.modules if m == "dilution_amd" or m.startswith("dilution_amd.")]:
             del sys.modules[mod]
+
+
+@pytest.mark.parametrize("version,said", [(4, "lacks dil_forward_rows"), (3, "has ABI 3, expected 4")])
+def test_another_build_is_an_explained_error(tmp_path, version, said):
+    """DILUTION_HIP_LIB naming a library of another ABI, or of this one without
+    the entry points added since: the package imports, HAS_HIP is False, and a
+    call says why."""
+    import subprocess
+    import sys
+
+    src, so = tmp_path / "old.c", tmp_path / "old.so"
+    src.write_text(f"int dil_abi_version(void) {{ return {version}; }}\n"
+                   + "\n".join(f"int {name}(void) {{ return 0; }}" for name in _declared_symbols()
+                               if name != "dil_abi_version" and not name.startswith("dil_forward_rows")))
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    code = """
+import torch
+from dilution import _hip, kernels
+assert not kernels.HAS_HIP
+x, r = torch.zeros(1, 1, 4, 16), torch.zeros(1, 4)
+for call in (_hip.lib, lambda: kernels._backward([x, x, x, x, r, r, r, r, x], x, "bf16", kernels._PRODUCTION)):
+    try:
+        call()
+    except RuntimeError as exc:
+        assert _hip.load_error() in str(exc), exc
+print(_hip.load_error())
+"""
+    env = dict(os.environ, DILUTION_HIP_LIB=str(so), PYTHONPATH=os.path.join(ROOT, "dilution-attention_amd"))
+    out = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True)
+    assert out.returncode == 0 and said in out.stdout, out.stdout + out.stderr
