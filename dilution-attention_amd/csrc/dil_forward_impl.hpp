@@ -1102,8 +1102,8 @@ inline int64_t keyout_partial_bytes(int kw, int64_t n, int64_t C, int64_t Tk, in
 // steps over 256 CUs; the reduction reads the partials at 4.5 TB/s.  Measured, us
 // (pass + reduction, 16 / 8 waves): B2 H8 T4096 268 / 216, B3 H5 T1357 96 / 78,
 // B2 H4 T2048 135 / 101, B8 H16 T2048 212 / 252, B32 H12 T1024 215 / 240,
-// B1 H16 T16384 1336 / 1697.  (Calls of few short rows take the three passes
-// now, few_short_rows: the pass meets rows up to 2048 with many slices only.)
+// B1 H16 T16384 1336 / 1697.  (Calls of few short rows take the three passes,
+// few_short_rows: of rows from 193 to 2048 keys the pass meets many slices only.)
 inline int keyout_waves(int64_t n, int64_t C, int64_t Tk, int D) {
   auto us = [&](int kw, double step, double full_step) {
     const double walk = static_cast<double>((C + kTileQ - 1) / kTileQ) * step;

@@ -355,7 +355,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, Maybe> prefill_chunk(
   at::Tensor out = into ? *into : at::empty({batch, heads, chunk, d}, o);
   const at::Tensor orows = out.size(0) == sd.first && out.size(1) == sd.second ? out : out.view({sd.first, sd.second, chunk, d});
   at::Tensor rmax = at::empty({n, chunk}, o), rden = at::empty({n, chunk}, o), ssum = at::empty({n, chunk}, o);
-  // the key pass writes the checkpoints only for a caller that keeps them
+  // a caller that keeps no checkpoints passes none where the library needs none
   Maybe carry;
   if (keep_carry || !api.forward_key_pass(chunk, start, static_cast<int>(d), tc, prec))
     carry = at::empty({n, (chunk + kCheckpointRows - 1) / kCheckpointRows, start + chunk}, o);

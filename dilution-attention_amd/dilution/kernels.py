@@ -163,7 +163,7 @@ def _native():
 
 def _raw_stream(x: torch.Tensor) -> int:
     """The current stream of x's device, as its raw handle (0 for a CPU
-    tensor, which the native checks refuse)."""
+    tensor: the native calls check every tensor's device)."""
     idx = x.get_device()
     return torch._C._cuda_getCurrentRawStream(idx) if idx >= 0 else 0
 
@@ -209,10 +209,15 @@ def dilution_attention_forward(
     entries past them are left unwritten, as in the reference
     (kernels.py:353-354; its tests read ``carry[:, b, :end]`` only).  Without
     return_aux no checkpoint is kept: the key-parallel pass (bf16 operands,
-    head_dim 64) writes none, and the three-pass forward processes the
-    (batch, head) slices in groups sized so its (rows, T/32, T) fp32
-    checkpoint scratch stays under scratch_budget_gib; slices are independent,
-    so results are identical either way.
+    head_dim 64) writes none, few short rows of that kind hold theirs in the
+    workspace (at most 32 MiB), and elsewhere the three-pass forward processes
+    the (batch, head) slices in groups sized so its (rows, T/32, T) fp32
+    checkpoint scratch stays under scratch_budget_gib.  The results are the same
+    bits with and without aux and in groups of any size.
+
+    A slice's results are not the same bits in calls of different B * H: the
+    size of a call picks the order of some sums (rows of at most 2048 keys, and
+    at any length for other than bf16 operands at head_dim 64).
     """
     _precision_code(dot_precision)
     out, rmax, rden, ssum, total, pk, carry = _native().forward(
@@ -313,9 +318,9 @@ def dilution_prefill_chunk(
     (entries beyond start + C are not touched).  Returns the chunk's outputs
     (B, H, C, D) fp32, and with return_aux the chunk's rmax/rden/ssum/carry.
     Chaining chunks reproduces ``dilution_attention_forward`` row for row and
-    its ``aux["committed_total"]``.  ``_out`` (a (B, H, C, D) view that
-    ``_strided_rows`` accepts, any float dtype) takes the outputs in place of a
-    new fp32 tensor.
+    its ``aux["committed_total"]`` to rounding.  ``_out`` (a (B, H, C, D) view
+    in fp32, bf16 or fp16 that ``dil_rows`` can describe) takes the outputs in
+    place of a new fp32 tensor.
     """
     _precision_code(dot_precision)
     out, rmax, rden, ssum, carry = _native().prefill_chunk(

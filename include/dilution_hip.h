@@ -32,6 +32,11 @@
  *   - The key-parallel forward's workspace holds at most 24 GiB of output
  *     partials; a call whose slices need more runs over them in batches, so
  *     the forward workspace stays bounded at any batch size.
+ *   - A slice's results may depend in their last bits on how many slices are in
+ *     the call: the size of a call picks the order of some sums (the forward's
+ *     for rows of at most 2048 keys, and at any length for operands other than
+ *     bf16 at head_dim 64 and for prefill chunks that start off the multiples of
+ *     512; dk's up to head_dim 128; the decode step's).
  *   - The forward's and the prefill's workspace queries are not monotone in the
  *     slice count: a smaller call may be quicker with up to 1 GiB of partials
  *     that a larger one has no use for.  A workspace sized for more slices of
@@ -75,10 +80,12 @@ typedef struct dil_rows {
 
 /*
  * Whether a dil_forward call (start = 0, chunk = seq) or a dil_prefill_chunk
- * call of this shape takes the key-parallel output pass: 1 or 0.  Its demand
- * checkpoints are an output only, so such a call may pass carry = NULL (an
- * inference forward or a prefill chunk that keeps no aux); the three-pass
- * forward reads the checkpoints it writes and needs the array.  No reference
+ * call of this shape may pass carry = NULL (an inference forward or a prefill
+ * chunk that keeps no aux): 1 or 0.  1 where the key-parallel output pass, whose
+ * demand checkpoints are an output only, can run; few short rows of such shapes
+ * run the three-pass forward, with their checkpoints in the workspace when the
+ * caller gives no array.  Elsewhere the three-pass forward reads the checkpoints
+ * that it writes and needs the array.  No reference
  * counterpart: the reference's forward always writes its carry
  * (src/dilution/kernels.py:349-355).  Reads DILUTION_FORWARD_KEY_PASS as the
  * entry points do.
@@ -101,9 +108,8 @@ int dil_forward_key_pass(int64_t chunk, int64_t start, int head_dim, int dtype, 
  *            written for the block's causal keys j < 32*(b+1) only: the
  *            future triangle is left unwritten and never read (as the
  *            reference leaves it, kernels.py:353-354, test_kernels.py:143-149).
- *            May be NULL when dil_forward_key_pass(seq, 0, ...) is 1: then no
- *            checkpoint is written (outputs, statistics and totals are the
- *            same bits).
+ *            May be NULL when dil_forward_key_pass(seq, 0, ...) is 1: then none
+ *            is kept (outputs, statistics and totals are the same bits).
  * committed_total: (n, seq) float32 column totals of p (the decode demand).
  * pk:        (n, seq, head_dim) float32 (p @ k)/sqrt(head_dim), or NULL.
  */

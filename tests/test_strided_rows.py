@@ -44,7 +44,7 @@ def _inputs(shape, dtype, device="cuda"):
 
 @pytest.mark.parametrize("layout", list(LAYOUTS))
 def test_rule_matches_the_library(layout):
-    """_strided_rows says which views dil_forward_rows takes: the library's
+    """strided_rows says which views dil_forward_rows takes: the library's
     own check refuses the others (-4) before any launch, and passes the
     accepted ones on to its next check (a missing output, also -4, or a
     workspace that is too small, -3)."""
