@@ -1127,14 +1127,10 @@ inline bool keyout_eligible(int64_t C, int64_t Tk, int64_t q0, int D, int prec, 
 // 125 / 153, B4 H16 T1024 52 / 69, B16 H16 T256 26 / 31; beyond 2^17 tokens the
 // lead is gone (B8 H16 T2048 222 + 9 of V^T / 208).  Rows of more than 2048 keys
 // keep the key pass (its bits: a prefix has those of the whole sequence).
-// Without pk the three-pass forward's V^T is a launch of its own (~5 us): rows of
-// up to 192 keys do not earn it back, rows of up to 256 only where the walks are
-// split (a call without aux, us, key pass / three passes: 4 slices of 160 keys
-// 19.4 / 22.1, 200 22.2 / 21.5, 64 slices of 128 17.1 / 17.8, 200 23.7 / 20.6, 256
-// 25.0 / 22.0; 128 slices of 200 25.6 / 29.4).
-// The rule does not ask for pk: a call gives the same bits with and without it.
-inline bool few_short_rows(int64_t n, int64_t Tk) {
-  return Tk > 192 && Tk <= 2048 && n * Tk <= (int64_t{1} << (Tk <= 256 ? 14 : 17));
+// Without pk the three-pass forward's V^T is a launch of its own (~5 us), which
+// rows of up to 256 keys do not earn back.
+inline bool few_short_rows(int64_t n, int64_t Tk, bool pk) {
+  return Tk <= 2048 && n * Tk <= (int64_t{1} << 17) && (pk || Tk > 256);
 }
 // slices per key-pass batch: all of them when their partials fit the budget,
 // else as many batches as the budget needs, of equal size (a last batch of a
@@ -1168,7 +1164,7 @@ FwdWorkspace fwd_layout(int64_t n, int64_t C, int64_t Tk, int D, int dtype, int 
   w.total = w.op;
   // the key pass's partials, when a chunk of this shape can take it (every
   // call is a chunk of rows [Tk - C, Tk) against keys [0, Tk))
-  if (keyout_eligible(C, Tk, Tk - C, D, prec, key_pass) && few_short_rows(n, Tk)) {
+  if (keyout_eligible(C, Tk, Tk - C, D, prec, key_pass) && few_short_rows(n, Tk, want_pk != 0)) {
     // the three-pass forward's checkpoints, for a caller that keeps none
     w.total = w.carry + align_up(static_cast<size_t>(4 * n * ((C + kTileQ - 1) / kTileQ) * Tk));
   } else if (keyout_eligible(C, Tk, Tk - C, D, prec, key_pass)) {
@@ -1209,7 +1205,7 @@ int launch_forward(const ForwardArgs& a) {
   constexpr bool kKeyPassBuilt =
       std::is_same_v<CT, __bf16> && D == 64 && BID == BID_SOFTMAX && SHARE == SHARE_INCL;
   const bool could = kKeyPassBuilt && keyout_eligible(a.C, a.Tk, a.q0, D, kOperandPrec<CT>, a.key_pass);
-  const bool key_pass = could && !few_short_rows(a.n, a.Tk);
+  const bool key_pass = could && !few_short_rows(a.n, a.Tk, a.pk != nullptr);
   const bool v_rows = key_pass && !convert;
 
   // operands in the compute type; V^T (and K^T) tiles
