@@ -1103,7 +1103,7 @@ inline int64_t keyout_partial_bytes(int kw, int64_t n, int64_t C, int64_t Tk, in
 // (pass + reduction, 16 / 8 waves): B2 H8 T4096 268 / 216, B3 H5 T1357 96 / 78,
 // B2 H4 T2048 135 / 101, B8 H16 T2048 212 / 252, B32 H12 T1024 215 / 240,
 // B1 H16 T16384 1336 / 1697.  (Calls of few short rows take the three passes,
-// few_short_rows: of rows from 193 to 2048 keys the pass meets many slices only.)
+// few_short_rows: of rows from 257 to 2048 keys the pass meets many slices only.)
 inline int keyout_waves(int64_t n, int64_t C, int64_t Tk, int D) {
   auto us = [&](int kw, double step, double full_step) {
     const double walk = static_cast<double>((C + kTileQ - 1) / kTileQ) * step;
@@ -1128,7 +1128,11 @@ inline bool keyout_eligible(int64_t C, int64_t Tk, int64_t q0, int D, int prec, 
 // lead is gone (B8 H16 T2048 222 + 9 of V^T / 208).  Rows of more than 2048 keys
 // keep the key pass (its bits: a prefix has those of the whole sequence).
 // Without pk the three-pass forward's V^T is a launch of its own (~5 us), which
-// rows of up to 256 keys do not earn back.
+// rows of up to 256 keys do not earn back: there a call that keeps pk for a backward
+// and one that does not differ by rounding.  Both on the key pass would cost the
+// training call precision (bf16 partials: largest error 5.0e-3 instead of 2.4e-3 at
+// T96), both on three passes the other call 3 to 9 us (4 slices of 64 rows 14.5 ->
+// 17.7, 160 of 256 30.5 -> 39.3).
 inline bool few_short_rows(int64_t n, int64_t Tk, bool pk) {
   return Tk <= 2048 && n * Tk <= (int64_t{1} << 17) && (pk || Tk > 256);
 }

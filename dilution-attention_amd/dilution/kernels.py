@@ -213,7 +213,9 @@ def dilution_attention_forward(
     workspace (at most 32 MiB), and elsewhere the three-pass forward processes
     the (batch, head) slices in groups sized so its (rows, T/32, T) fp32
     checkpoint scratch stays under scratch_budget_gib.  The results are the same
-    bits with and without aux and in groups of any size.
+    bits with and without return_aux and in groups of any size; a call that
+    autograd keeps for a backward differs by rounding from one without at up to
+    256 rows (bf16 operands, head_dim 64).
 
     A slice's results are not the same bits in calls of different B * H: the
     size of a call picks the order of some sums (rows of at most 2048 keys, and

@@ -109,7 +109,9 @@ int dil_forward_key_pass(int64_t chunk, int64_t start, int head_dim, int dtype, 
  *            future triangle is left unwritten and never read (as the
  *            reference leaves it, kernels.py:353-354, test_kernels.py:143-149).
  *            May be NULL when dil_forward_key_pass(seq, 0, ...) is 1: then none
- *            is kept (outputs, statistics and totals are the same bits).
+ *            is kept (outputs, statistics and totals are the same bits; with and
+ *            without pk they agree to rounding at up to 256 rows of bf16
+ *            operands at head_dim 64).
  * committed_total: (n, seq) float32 column totals of p (the decode demand).
  * pk:        (n, seq, head_dim) float32 (p @ k)/sqrt(head_dim), or NULL.
  */
