@@ -1620,6 +1620,10 @@ int launch_backward(const BackwardArgs& a) {
   char* ws = static_cast<char*>(a.workspace);
   hipStream_t st = static_cast<hipStream_t>(a.stream);
   const bool convert = a.dtype != ctc;
+  // rows of q, k and v head_dim apart (converted ones are)
+  constexpr bool kStridedBuilt = is_production<BID, SHARE>() && D <= 128;
+  const bool rows_flat = convert || (a.qv.sr == D && a.kv.sr == D && a.vv.sr == D);
+  if (!kStridedBuilt && !rows_flat) return kErrShape;  // an argument error: before any launch
   const int64_t t_pad = pad64(a.T);
   const int64_t sn = a.T * D;
 
@@ -1690,8 +1694,7 @@ int launch_backward(const BackwardArgs& a) {
   });
   const int nkt = static_cast<int>((a.T + kTileK - 1) / kTileK);
   P.n = a.n;
-  const bool rows_flat = P.qv.sr == D && P.kv.sr == D && P.vv.sr == D;
-  return with_rows<is_production<BID, SHARE>() && D <= 128>(rows_flat, [&](auto flat_tag) -> int {
+  return with_rows<kStridedBuilt>(rows_flat, [&](auto flat_tag) -> int {
   constexpr bool kFlat = decltype(flat_tag)::value;
   // the softmax-Jacobian correction of dk: split walks where they are few
   auto dk_correction = [&](BwdParams K) {

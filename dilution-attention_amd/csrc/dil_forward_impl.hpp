@@ -1198,6 +1198,10 @@ int launch_forward(const ForwardArgs& a) {
   char* ws = static_cast<char*>(a.workspace);
   hipStream_t st = static_cast<hipStream_t>(a.stream);
   const bool convert = a.dtype != kNativeDtype<CT>;
+  // rows of q, k and v head_dim apart (converted q and k are)
+  constexpr bool kStridedBuilt = is_production<BID, SHARE>() && D <= 128;
+  const bool flat = (convert || (a.qv.sr == D && a.kv.sr == D)) && a.vv.sr == D;
+  if (!kStridedBuilt && !flat) return kErrShape;       // an argument error: before any launch
   const int64_t tk_pad = pad64(a.Tk);
 
   CT* vt = reinterpret_cast<CT*>(ws + w.vt);
@@ -1266,10 +1270,9 @@ int launch_forward(const ForwardArgs& a) {
   P.lshift = log2f(a.var.shift);
 
   P.n = a.n;
-  const bool flat = P.qv.sr == D && P.kv.sr == D && P.vv.sr == D;
   P.groups = static_cast<int>((a.C + 4 * kTileQ - 1) / (4 * kTileQ));
   const dim3 grid(static_cast<unsigned>(xcd_grid(P.groups * a.n)));
-  const int strided = with_rows<is_production<BID, SHARE>() && D <= 128>(flat, [&](auto flat_tag) -> int {
+  const int strided = with_rows<kStridedBuilt>(flat, [&](auto flat_tag) -> int {
   constexpr bool kFlat = decltype(flat_tag)::value;
   // Few tiles: their walks split over a workgroup's waves.  Not above 2048 keys
   // where the key pass could run: there a slice's bits don't depend on how many

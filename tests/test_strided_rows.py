@@ -163,3 +163,23 @@ def test_one_row_prompts_and_chunks(dim, bid_kw):
         want, c0 = cache.begin_cache(*xs, capacity=12, chunk=chunk, **bid_kw)
         got, c1 = cache.begin_cache(*(LAYOUTS["packed"](x) for x in xs), capacity=12, chunk=chunk, **bid_kw)
         assert torch.equal(got, want) and torch.equal(c0["committed"], c1["committed"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim,bid", [(64, 1), (256, 0)])
+def test_refused_rows_launch_nothing(dim, bid):
+    """Strided rows where only the contiguous form is built are an argument
+    error (-4) of the C ABI before any launch, forward and backward."""
+    lib, n, t = _hip.lib(), 6, 40
+    x = LAYOUTS["packed"](torch.randn(2, 3, t, dim, device="cuda").to(torch.bfloat16))
+    flat = torch.empty(2, 3, t, dim, device="cuda", dtype=torch.bfloat16)
+    f32 = [torch.empty(n * t * max(dim, 64), device="cuda") for _ in range(7)]
+    ws = torch.empty(lib.dil_forward_workspace_bytes(n, t, dim, 1, 2, 1) + lib.dil_backward_workspace_bytes(n, t, dim, 1, 2),
+                     dtype=torch.uint8, device="cuda")
+    row, out, ptr = _rows(x), _rows(flat), [b.data_ptr() for b in f32]
+    stream = torch.cuda.current_stream().cuda_stream
+    with _hip.kernel_timing() as kt:
+        forward = lib.dil_forward_rows(row, row, row, 2, 3, t, dim, 1, 2, bid, 1, 1.0, *ptr, ws.data_ptr(), ws.numel(), stream)
+        backward = lib.dil_backward_rows(row, row, row, row, *ptr[:6], 2, 3, t, dim, 1, 1, 1, 2, bid, 1, 1.0, out, out, out,
+                                         ws.data_ptr(), ws.numel(), stream)
+    assert (forward, backward) == (-4, -4) and not kt.result
